@@ -945,7 +945,7 @@ def main() -> int:
             "roofline": {
                 "bound": "mfma", "achieved": round(tflops, 2), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(tflops / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": None,
-                "kernel": "one pkv_prefill_attn call = append_kernel + prefill_lds_kernel<2,4,4,1> (LDS-staged KV tiles in 4 stages, 128 query rows per workgroup); " + per_call,
+                "kernel": "one pkv_prefill_attn call = append_kernel + prefill_tile_kernel<128> (LDS-staged KV tiles, 128 query rows per workgroup); " + per_call,
                 "flops_per_call": flops_layer, "bytes_per_call": bytes_layer, "avg_call_us": round(call_us, 3),
                 "hbm_gbs": round(gbs, 1),
             },
@@ -980,7 +980,7 @@ def main() -> int:
                    "frac_unique": round(unique_layer / (c_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
                    "mfma_tflops": round(flops_layer / (c_us * 1e-6) / 1e12, 2),
                    "mfma_frac": round(flops_layer / (c_us * 1e-6) / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4),
-                   "kernels": "prefill_lds_kernel (prefix pass, key splits) + decode_lean_kernel<3> (suffixes) + "
+                   "kernels": "prefill_tile_kernel (prefix pass, key splits) + decode_lean_kernel<3> (suffixes) + "
                               "combine_lean_kernel; HIP events around graph replays"}
         # the same verify where the shared prefix dominates (8192-token prompt, suffixes <= 256)
         wl = workloads.config5(dev, seed=args.seed, prefix=8192, max_suffix=256)

@@ -404,13 +404,6 @@ constexpr float kRescaleSlack = 8.0f;
 #ifndef PKV_PREFILL_DEPTH
 #define PKV_PREFILL_DEPTH 1
 #endif
-// prefill's software pipeline, and the vector instructions between its interleaved MFMAs
-#ifndef PKV_PREFILL_PIPE
-#define PKV_PREFILL_PIPE 1
-#endif
-#ifndef PKV_PREFILL_PIPE_VALU
-#define PKV_PREFILL_PIPE_VALU 2
-#endif
 constexpr int kDecodeDepth = PKV_DECODE_DEPTH;
 constexpr int kPrefillDepth = PKV_PREFILL_DEPTH;
 
@@ -2653,58 +2646,24 @@ __global__ __launch_bounds__(64 * W) void prefill_kernel(const AttnParams p) {
   }
 }
 
-// ---------------------------------------------------------------------------------------------
-// Chunked prefill with LDS-staged KV tiles (head_dim 128, pages of >= 32 rows): grid (row block,
-// KV head, sequence).  The W waves of a workgroup own 16*NT consecutive query rows each (row =
-// j * g + head-in-group, so a block spans a few query positions of every head of the group) and
-// share each 32-token K / V tile of their KV head: the workgroup copies a tile into LDS once
-// (16 buffer loads of 1 KiB straight into LDS, 16 / W per wave) into one of NBUF stage buffers,
-// and every wave reads its MFMA operands from there (16-byte chunks XOR-swizzled per row: K rows
-// by swz as in the decode kernel, V rows by swz_v for the transpose reads).
-// The block walks keys up to its last row's last visible key; rows that see fewer keys are masked
-// inside the tiles that cross their limit.  No split-K: every wave writes its own rows.
-// ---------------------------------------------------------------------------------------------
-namespace pf {
-constexpr int HD = 128;
-constexpr int ROW = HD * 2;            // one KV head's slice of a token row: 256 B
-constexpr int TILE = 32;
-constexpr int KV_BYTES = TILE * ROW;   // 8 KiB of K (or V) per tile
-constexpr int BUF = 2 * KV_BYTES;      // K | V
-// 16-byte chunk swizzle of V row r (LDS chunk c holds global chunk c ^ swz_v(r)).  A transpose
-// read of V^T operand n touches, in each half wave, token rows 8 q + 4 h + j (j < 4, q one of two
-// adjacent values) at global chunks 2 n and 2 n + 1: bits 1..3 of the swizzle take 8 distinct
-// values over those rows, so the 8 chunk pairs fall in 8 different bank ranges.
-__device__ __forceinline__ int swz_v(int r) { return ((r & 3) << 1) | (((r >> 3) & 1) << 3); }
-}  // namespace pf
-
-template <int OPS, int NBUF>
-__device__ __forceinline__ void pf_wait(int ahead) {
-  // at most `ahead` later tiles' copies (OPS per tile for this wave) may stay in flight
-  static_assert(OPS * (NBUF - 1) <= 15, "vmcnt immediate");
-  switch (ahead) {
-    case 0: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-    case 1: __builtin_amdgcn_s_waitcnt(0x0F70 | OPS); break;
-    case 2: __builtin_amdgcn_s_waitcnt(0x0F70 | (NBUF > 2 ? 2 * OPS : OPS)); break;
-    default: __builtin_amdgcn_s_waitcnt(0x0F70 | (OPS * (NBUF - 1))); break;
-  }
-}
-
-// Online-softmax update of a wave's 16*NT prefill rows with one 32-token tile, arranged for
-// instruction-level parallelism across the N tiles: every S^T product first (NT x 2 independent
-// MFMA chains), then the softmax of all tiles with one wave-uniform rescale test, then every PV
-// product.  The row max is taken on raw scores (the scale is positive) and the scale is folded
-// into the exponent's FMA.  P is rounded to bf16 once (prefill has no MFMA headroom to spare).
-// The update itself, on ready operands: kr the tile's K rows (QK^T A operands), vt[n] the V^T
-// A operands (lane (i, q): 8 keys 8 q .. 8 q + 7 of one head-dim element per operand; which
-// element lane i holds in operand n is the caller's layout, and the accumulator row of that lane
-// follows it).
-// l_run is either a per-lane partial row sum (float: this lane's keys, summed over the four lanes
-// of a row at the end) or the whole row sum kept by the matrix cores (f32x4: P times a ones
-// operand, every element the row's sum, of the same bf16 P the PV product uses), which takes the
-// 16 additions per tile off the vector ALU for NT extra products.
-// S^T products of a tile: NT x 2 independent chains of 4 MFMAs over the head dimension.
-template <int NT>
-__device__ __forceinline__ void pf_qk(const u32x4 (&kr)[2][4], const bf16x8 (&qf)[NT][4], f32x4 (&s)[NT][2]) {
+// Verify tile update (decode_lean_kernel's NT > 1): the online-softmax update of a wave's 16*NT query
+// rows with one 32-token tile, arranged for instruction-level parallelism across the N tiles: every
+// S^T product first (NT x 2 independent MFMA chains), then the softmax of all tiles with one
+// wave-uniform rescale test, then every PV product.  The row max is taken on raw scores (the scale is
+// positive) and the scale is folded into the exponent's FMA.  P is rounded to bf16 once.
+// kr holds the tile's K rows (QK^T A operands); v_ops delivers vt[n], the V^T A operands (lane (i, q):
+// 8 keys 8 q .. 8 q + 7 of one head-dim element per operand; which element lane i holds in operand n
+// is the caller's layout, and the accumulator row of that lane follows it).  l_run is a per-lane
+// partial row sum (this lane's keys, summed over the four lanes of a row at the end).
+template <int NT, typename VOps>
+__device__ __forceinline__ void compute_tile_prefill_ops(const AttnParams& p, const u32x4 (&kr)[2][4], VOps&& v_ops,
+                                                         int T0, const bf16x8 (&qf)[NT][4], const int (&lim)[NT],
+                                                         int lim_min, float (&m_run)[NT], float (&l_run)[NT],
+                                                         f32x4 (&acc)[NT][8]) {
+  constexpr int DPL = 8;
+  const int lane = threadIdx.x & 63;
+  const int lq = lane >> 4;
+  f32x4 s[NT][2];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -2715,27 +2674,6 @@ __device__ __forceinline__ void pf_qk(const u32x4 (&kr)[2][4], const bf16x8 (&qf
         s[nt][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kr[a][kk]), qf[nt][kk],
                                                            s[nt][a], 0, 0, 0);
     }
-}
-
-// The rest of the update from the scores s: mask, rescale, P, row sums and PV.  With NEXT, the
-// next tile's S^T products (K operands kn, into sn) go out interleaved with this tile's
-// exponentials, one MFMA between every few vector instructions: a wave issues in order and its
-// next MFMA waits for the matrix pipe, so products placed back to back would hold the softmax
-// behind them, while interleaved the two pipes work at once.
-// PRIO: the PV products issue at raised wave priority.  With two waves per SIMD (prefill), the
-// wave holding its PV products then wins the issue slots over the other wave's exponentials
-// whenever the matrix pipe can take a product, so the two waves drift into opposite phases
-// instead of queueing for the same pipe (prefill-4096 142.7 -> 132.8 us; verify, at one wave per
-// SIMD, 57.7 -> 58.0, so it stays off there).
-template <int NT, bool NEXT, bool PRIO = false, typename LT, typename VOps>
-__device__ __forceinline__ void pf_softmax_pv(const AttnParams& p, f32x4 (&s)[NT][2], const u32x4 (&kn)[2][4],
-                                              f32x4 (&sn)[NT][2], VOps&& v_ops, int T0, const bf16x8 (&qf)[NT][4],
-                                              const int (&lim)[NT], int lim_min, float (&m_run)[NT],
-                                              LT (&l_run)[NT], f32x4 (&acc)[NT][8]) {
-  constexpr bool kLByMfma = std::is_same<LT, f32x4>::value;
-  constexpr int DPL = 8;
-  const int lane = threadIdx.x & 63;
-  const int lq = lane >> 4;
   if (T0 + 31 > lim_min) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -2778,59 +2716,19 @@ __device__ __forceinline__ void pf_softmax_pv(const AttnParams& p, f32x4 (&s)[NT
     for (int e = 0; e < 8; e += 2) {
       const float p0 = fast_exp2(fmaf(s[nt][e >> 2][e & 3], p.scale_log2, neg_m));
       const float p1 = fast_exp2(fmaf(s[nt][e >> 2][(e & 3) + 1], p.scale_log2, neg_m));
-      if constexpr (!kLByMfma) psum += p0 + p1;
+      psum += p0 + p1;
       pk[e >> 1] = pack_bf16x2(p0, p1);
     }
-    if constexpr (!kLByMfma) l_run[nt] += psum;
+    l_run[nt] += psum;
     pb[nt] = __builtin_bit_cast(bf16x8, pk);
-  }
-  if constexpr (NEXT) {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int a = 0; a < 2; ++a) sn[nt][a] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-          sn[nt][a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kn[a][kk]), qf[nt][kk],
-                                                              sn[nt][a], 0, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 8 * NT; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, PKV_PREFILL_PIPE_VALU, 0);  // then vector ALU work
-    }
-  }
-  if constexpr (kLByMfma) {
-    const u32x4 one2 = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};  // bf16 1.0 pairs
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      l_run[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, one2), pb[nt], l_run[nt], 0, 0, 0);
   }
   bf16x8 vt[DPL];
   v_ops(vt);
-  if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int n = 0; n < DPL; ++n)
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
       acc[nt][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[n], pb[nt], acc[nt][n], 0, 0, 0);
-  if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
-}
-
-template <int NT, typename LT, typename VIssue, typename VOps>
-__device__ __forceinline__ void compute_tile_prefill_ops(const AttnParams& p, const u32x4 (&kr)[2][4],
-                                                         VIssue&& v_issue, VOps&& v_ops, int T0,
-                                                         const bf16x8 (&qf)[NT][4],
-                                                         const int (&lim)[NT], int lim_min, float (&m_run)[NT],
-                                                         LT (&l_run)[NT], f32x4 (&acc)[NT][8]) {
-  f32x4 s[NT][2];
-  pf_qk<NT>(kr, qf, s);
-  v_issue();
-  f32x4 sn_unused[NT][2];
-  pf_softmax_pv<NT, false>(p, s, kr, sn_unused, v_ops, T0, qf, lim, lim_min, m_run, l_run, acc);
 }
 
 // The same update on a tile read row-wise (KVTile): V^T operand n of lane (i, q) is head-dim
@@ -2850,7 +2748,7 @@ __device__ __forceinline__ void compute_tile_prefill(const AttnParams& p, const 
       vt[n] = __builtin_bit_cast(bf16x8, pk);
     }
   };
-  compute_tile_prefill_ops<NT>(p, tl.kr, [] {}, v_ops, T0, qf, lim, lim_min, m_run, l_run, acc);
+  compute_tile_prefill_ops<NT>(p, tl.kr, v_ops, T0, qf, lim, lim_min, m_run, l_run, acc);
 }
 
 // The same update on a tile whose V^T operands came from transpose reads (rows_read_tile_vt).
@@ -2864,7 +2762,7 @@ __device__ __forceinline__ void compute_tile_prefill_vt(const AttnParams& p, con
     for (int n = 0; n < 8; ++n)
       vt[n] = __builtin_bit_cast(bf16x8, u32x4{tl.vr[n].w[0], tl.vr[n].w[1], tl.vr[n].w[2], tl.vr[n].w[3]});
   };
-  compute_tile_prefill_ops<NT>(p, tl.kr, [] {}, v_ops, T0, qf, lim, lim_min, m_run, l_run, acc);
+  compute_tile_prefill_ops<NT>(p, tl.kr, v_ops, T0, qf, lim, lim_min, m_run, l_run, acc);
 }
 
 // Input check of a cascade launch, by one wave: sequences b0..b1 must list sequence 0's first
@@ -2889,339 +2787,7 @@ __device__ __forceinline__ void cascade_check_sharing(const AttnParams& p, int b
   if (__any(bad) && lane == 0) flag_status(p.status, PKV_STATUS_SHARED_PREFIX);
 }
 
-// CASCADE: the shared-prefix pass of a cascade launch.  Grid (row blocks of the whole batch's
-// query rows, KV heads, key splits); block-table row 0 holds the shared pages; split z covers
-// tiles [z chunk, (z + 1) chunk) of the k0 shared keys, which every row sees whole; the result is
-// a partial (fp16 O / l and fp32 log-sum-exp) in workspace slot 2 G + b S + z of each row.
-template <int NT, int W, int NBUF, int SUB, bool CASCADE = false>
-__global__ __launch_bounds__(64 * W) void prefill_lds_kernel(const AttnParams p) {
-  constexpr int HD = pf::HD;
-  constexpr int DPL = HD / 16;
-  constexpr int OPS = 16 / W * SUB;  // copies per wave per stage (SUB tiles of 32 tokens)
-  static_assert(16 % W == 0, "waves must split the 16 copies of a tile");
-  __shared__ __attribute__((aligned(16))) char lds[NBUF * SUB * pf::BUF];
-
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int li = lane & 15;
-  const int lq = lane >> 4;
-  int b, h, xblk;
-  int c, L;
-  const int R_all = CASCADE ? p.batch * p.R : p.R;  // query rows of the launch's row space
-  int t_first = 0;                                  // first tile of this workgroup's key range
-  int n_tiles;
-  if constexpr (CASCADE) {
-    xblk = blockIdx.x;
-    h = blockIdx.y;
-    b = 0;
-    c = 0;
-    L = p.k0;
-    const int n_shared = p.k0 / pf::TILE;
-    const int chunk = (n_shared + int(gridDim.z) - 1) / int(gridDim.z);
-    t_first = int(blockIdx.z) * chunk;
-    n_tiles = min(chunk, n_shared - t_first);
-  } else {
-    prefill_item(p, b, h, xblk);
-    seq_lengths(p, b, c, L);
-  }
-  SeqView sv;
-  sv.b = b;
-  sv.h = h;
-  sv.c = c;
-  sv.t_end = L;
-  sv.bt = p.block_table + int64_t(b) * p.bt_stride;
-
-  const int blk_row0 = xblk * W * 16 * NT;
-  if (blk_row0 >= R_all) return;
-  const int row0 = blk_row0 + wave * 16 * NT;
-  // the block's last row sees the most keys (rows increase with j)
-  const int blk_last = min(blk_row0 + W * 16 * NT, R_all) - 1;
-  if constexpr (CASCADE) {
-    if (blockIdx.z == 0 && h == 0) cascade_check_sharing(p, blk_row0 / p.R, blk_last / p.R);
-    if (n_tiles <= 0) n_tiles = 0;
-  } else {
-    const int t_stop = p.causal ? min(L, L - p.s_q + blk_last / p.g + 1) : L;
-    n_tiles = t_stop > 0 ? (t_stop + pf::TILE - 1) / pf::TILE : 0;
-  }
-  const int n_stages = (n_tiles + SUB - 1) / SUB;
-
-  bf16x8 qf[NT][HD / 32];
-  int lim[NT];
-  if constexpr (CASCADE)
-    load_q_batch_rows<HD, NT>(p, h, row0, p.k0 - 1, qf, lim);
-  else
-    load_q<HD, NT>(p, sv, L, row0, qf, lim);
-  // Q is in registers before any tile copy goes out: the tile loop's waits then never have to
-  // account for it (the copy pipeline's own waits are the explicit pf_wait ones)
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  int lim_min = 0x7fffffff;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) lim_min = min_real_limit(lim_min, lim[nt]);
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) lim_min = min(lim_min, __shfl_xor(lim_min, off, 64));
-  lim_min = __builtin_amdgcn_readfirstlane(lim_min);
-
-  BtWindow btw;
-  bt_window_load(p, sv, (t_first * pf::TILE) >> p.log2_page, btw);
-  const int row_elems = p.n_kv * HD;
-  // Stage st holds tiles SUB*st .. SUB*st + SUB-1 (the last stage repeats its last real tile so
-  // every stage issues the same number of copies).  Copy instruction i of a tile: K (i < 8) or V
-  // rows 4 (i % 8) .. +3, lane l -> row + l / 16, LDS chunk l % 16 <- global chunk (l % 16) ^ swizzle
-  // (swz for K rows, swz_v for V rows).
-  // The copies are buffer loads: a tile's K and V rows of this head are one buffer each (base and
-  // range in scalar registers), and each lane's byte offset inside it is the same for every tile.
-  uint32_t voff[16 / W];
-#pragma unroll
-  for (int k = 0; k < 16 / W; ++k) {
-    const int i = wave + k * W;
-    const int r = 4 * (i & 7) + (lane >> 4);
-    voff[k] = uint32_t(r * row_elems + ((lane & 15) ^ (i < 8 ? rows::swz(r) : pf::swz_v(r))) * 8) * 2u;
-  }
-  const int tile_bytes = pf::TILE * row_elems * 2;
-  auto issue = [&](int st) {
-    char* stage = lds + (st % NBUF) * SUB * pf::BUF;
-#pragma unroll
-    for (int u = 0; u < SUB; ++u) {
-      const int T0 = (t_first + min(st * SUB + u, n_tiles - 1)) * pf::TILE;
-      const int pid = bt_page(p, sv, T0 >> p.log2_page, btw);
-      const bool ok = unsigned(pid) < unsigned(p.num_pages);
-      if (!ok && T0 < L && lane == 0) flag_status(p.status, PKV_STATUS_BAD_PAGE);
-      const int64_t off = int64_t(ok ? pid : 0) * p.page_stride +
-                          int64_t(T0 & ((1 << p.log2_page) - 1)) * row_elems + h * HD;
-      char* buf = stage + u * pf::BUF;
-#pragma unroll
-      for (int k = 0; k < 16 / W; ++k) {
-        const int i = wave + k * W;
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            uniform_ptr((i < 8 ? p.k_cache : p.v_cache) + off), 0, tile_bytes, 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs,
-                                                 (rows::lds_void*)(buf + (i >= 8 ? pf::KV_BYTES : 0) + (i & 7) * 1024),
-                                                 16, int(voff[k]), 0, 0, 0);
-      }
-    }
-  };
-  // NBUF == 2: stage st + 2 is issued into st's buffer once every wave has read it (a second
-  // barrier per tile).  NBUF >= 3: stage st + NBUF - 1 is issued into the buffer of stage st - 1
-  // right after the tile's first barrier, which every wave passes only after it has consumed
-  // stage st - 1: one barrier per tile, and NBUF - 1 stages in flight during the compute.
-  constexpr bool kOneBarrier = NBUF >= 3;
-  for (int st = 0; st < (kOneBarrier ? NBUF - 1 : NBUF) && st < n_stages; ++st) issue(st);
-  // V^T operands come from LDS transpose reads (ds_read_b64_tr_b16): in each 16-lane group, lane
-  // 4 j + c names 4 consecutive elements of row j of a 4 x 16 block of 16-bit values and receives
-  // column (its index in the group) of that block.  Operand n of lane (li, lq) is head-dim element
-  // 16 n + li over keys 8 lq .. 8 lq + 7: two reads, of token rows 8 lq + j and 8 lq + 4 + j (the
-  // same swizzle, 4 rows further), each lane naming elements 16 n + 4 c .. + 3.  vtr[n] is that
-  // lane's byte offset inside a tile's V rows, the same for every tile.
-  uint32_t vtr[8];
-  {
-    const int t = 8 * lq + (li >> 2);
-    const int c = li & 3;
-#pragma unroll
-    for (int n = 0; n < 8; ++n)
-      vtr[n] = uint32_t(t * pf::ROW + (((2 * n + (c >> 1)) ^ pf::swz_v(t)) << 4) + 8 * (c & 1));
-  }
-
-  float m_run[NT];
-  f32x4 l_run[NT];  // row sums kept by the matrix cores (every element the row's sum)
-  f32x4 acc[NT][DPL];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    m_run[nt] = -INFINITY;
-    l_run[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int n = 0; n < DPL; ++n) acc[nt][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  // Software pipeline (one tile per stage, NBUF >= 3): tile t's softmax and PV products run with
-  // tile t + 1's S^T products interleaved, so every iteration first waits for stage t + 1.  After
-  // that wait's barrier no wave reads stage t - 1 any more (its K went into the products of
-  // iteration t - 2, its V into those of t - 1), so stage t + NBUF - 1 is issued into its buffer.
-  constexpr bool kPipe = kOneBarrier && SUB == 1 && PKV_PREFILL_PIPE;
-  if constexpr (kPipe) {
-    auto read_k = [&](int t, u32x4 (&kr)[2][4]) {
-      const char* buf = lds + (t % NBUF) * pf::BUF;
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        const int r = 8 * (li >> 2) + 4 * a + (li & 3);
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-          kr[a][kk] = *reinterpret_cast<const u32x4*>(buf + r * pf::ROW + (((4 * kk + lq) ^ rows::swz(r)) << 4));
-      }
-    };
-    f32x4 s[NT][2];
-    pf_wait<OPS, NBUF>(min(NBUF - 2, n_stages - 1));
-    raw_barrier();
-    if (row0 < R_all && n_tiles > 0) {
-      u32x4 kr[2][4];
-      read_k(0, kr);
-      pf_qk<NT>(kr, qf, s);
-    }
-    // tile t's update, with tile t + 1's products when NEXT
-    auto step = [&](int t, auto next) {
-      constexpr bool NEXT = decltype(next)::value;
-      if (row0 >= R_all) return;
-      const int T0 = (t_first + t) * pf::TILE;
-      const uint32_t vrows = lds_addr(lds + (t % NBUF) * pf::BUF + pf::KV_BYTES);
-      u32x2 vlo[8], vhi[8];
-      // the V^T reads go out before the next tile's K reads, so the compiler's own wait for
-      // those (it does not count these) also covers them
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int n = 0; n < 8; ++n) {
-        vlo[n] = lds_read_tr16_issue<0>(vrows + vtr[n]);
-        vhi[n] = lds_read_tr16_issue<4 * pf::ROW>(vrows + vtr[n]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      auto v_ops = [&](bf16x8 (&vt)[8]) {
-        lds_tr_wait(vlo, vhi);
-        u32x4 vw[8];
-#pragma unroll
-        for (int n = 0; n < 8; ++n) vw[n] = u32x4{vlo[n][0], vlo[n][1], vhi[n][0], vhi[n][1]};
-        if (T0 + pf::TILE > L) {
-          // keys past the sequence: P = 0 must not meet a stale NaN (word w holds keys 2 w, 2 w + 1)
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            const int k = T0 + 8 * lq + 2 * w;
-            const uint32_t keep = (k < L ? 0x0000FFFFu : 0u) | (k + 1 < L ? 0xFFFF0000u : 0u);
-#pragma unroll
-            for (int n = 0; n < 8; ++n) vw[n][w] &= keep;
-          }
-        }
-#pragma unroll
-        for (int n = 0; n < 8; ++n) vt[n] = __builtin_bit_cast(bf16x8, vw[n]);
-      };
-      u32x4 kn[2][4];
-      f32x4 sn[NT][2];
-      if constexpr (NEXT) read_k(t + 1, kn);
-      pf_softmax_pv<NT, NEXT, true>(p, s, kn, sn, v_ops, T0, qf, lim, lim_min, m_run, l_run, acc);
-      if constexpr (NEXT) {
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-          for (int a = 0; a < 2; ++a) s[nt][a] = sn[nt][a];
-      }
-    };
-    for (int t = 0; t + 1 < n_tiles; ++t) {
-      pf_wait<OPS, NBUF>(min(NBUF - 3, n_stages - 2 - t));
-      raw_barrier();
-      if (t + NBUF - 1 < n_stages) issue(t + NBUF - 1);
-      step(t, std::true_type{});
-    }
-    if (n_tiles > 0) step(n_tiles - 1, std::false_type{});
-  } else {
-    for (int st = 0; st < n_stages; ++st) {
-      if constexpr (kOneBarrier) {
-        pf_wait<OPS, NBUF>(min(NBUF - 2, n_stages - 1 - st));
-        raw_barrier();
-        if (st + NBUF - 1 < n_stages) issue(st + NBUF - 1);
-      } else {
-        pf_wait<OPS, NBUF>(min(NBUF - 1, n_stages - 1 - st));
-        raw_barrier();
-      }
-  #pragma unroll
-      for (int u = 0; u < SUB; ++u) {
-        const int t = st * SUB + u;
-        if (t >= n_tiles) break;
-        const int T0 = (t_first + t) * pf::TILE;
-        const char* buf = lds + ((st % NBUF) * SUB + u) * pf::BUF;
-        u32x4 kr[2][4];
-  #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          const int r = 8 * (li >> 2) + 4 * a + (li & 3);
-  #pragma unroll
-          for (int kk = 0; kk < 4; ++kk)
-            kr[a][kk] = *reinterpret_cast<const u32x4*>(buf + r * pf::ROW + (((4 * kk + lq) ^ rows::swz(r)) << 4));
-        }
-        // the V^T reads go out once the QK products are issued (so the compiler's waits for the K
-        // reads, which do not count these, stay exact) and are waited for just before the PV
-        // products (lds_tr_wait): their latency hides behind the QK products and the softmax
-        const uint32_t vrows = lds_addr(buf + pf::KV_BYTES);
-        u32x2 vlo[8], vhi[8];
-        auto v_issue = [&] {
-          __builtin_amdgcn_sched_barrier(0);
-  #pragma unroll
-          for (int n = 0; n < 8; ++n) {
-            vlo[n] = lds_read_tr16_issue<0>(vrows + vtr[n]);
-            vhi[n] = lds_read_tr16_issue<4 * pf::ROW>(vrows + vtr[n]);
-          }
-        };
-        auto v_ops = [&](bf16x8 (&vt)[8]) {
-          lds_tr_wait(vlo, vhi);
-          u32x4 vw[8];
-  #pragma unroll
-          for (int n = 0; n < 8; ++n) vw[n] = u32x4{vlo[n][0], vlo[n][1], vhi[n][0], vhi[n][1]};
-          if (T0 + pf::TILE > L) {
-            // keys past the sequence: P = 0 must not meet a stale NaN (word w holds keys 2 w, 2 w + 1)
-  #pragma unroll
-            for (int w = 0; w < 4; ++w) {
-              const int k = T0 + 8 * lq + 2 * w;
-              const uint32_t keep = (k < L ? 0x0000FFFFu : 0u) | (k + 1 < L ? 0xFFFF0000u : 0u);
-  #pragma unroll
-              for (int n = 0; n < 8; ++n) vw[n][w] &= keep;
-            }
-          }
-  #pragma unroll
-          for (int n = 0; n < 8; ++n) vt[n] = __builtin_bit_cast(bf16x8, vw[n]);
-        };
-        if (row0 < R_all) compute_tile_prefill_ops<NT>(p, kr, v_issue, v_ops, T0, qf, lim, lim_min, m_run, l_run, acc);
-      }
-      if constexpr (!kOneBarrier) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of the stage are done
-        raw_barrier();                       // the stage's buffer is free
-        if (st + NBUF < n_stages) issue(st + NBUF);
-      }
-    }
-  }
-  if (row0 >= R_all) return;
-  if constexpr (CASCADE) {
-    // the split's partial of every row: fp16 O / l and the log-sum-exp, as the balanced kernel
-    // writes its partials
-    const uint32_t lse0 = uint32_t(p.ws_ml - p.ws_o) * 4u;
-    const __amdgpu_buffer_rsrc_t rs = ws_rsrc(p);
-    bool ovf = false;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int ra = row0 + li + 16 * nt;
-      const float lsum = l_run[nt][0];
-      if (ra < R_all) {
-        const int br = ra / p.R;
-        const int rr = ra - br * p.R;
-        const int slot = 2 * p.lean_grid + br * p.cascade_splits + int(blockIdx.z);
-        const uint32_t row = uint32_t((slot * rows::NKV + h) * p.R + rr);
-        const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-        // accumulator n of lane (li, lq) holds head-dim elements 16 n + 4 lq .. + 3
-#pragma unroll
-        for (int n = 0; n < DPL; ++n) {
-          const f32x4 o = acc[nt][n] * inv;
-          ovf = ovf || f16_overflows(o[0], o[1]) || f16_overflows(o[2], o[3]);
-          const u32x2 ov = {pack_f16x2(o[0], o[1]), pack_f16x2(o[2], o[3])};
-          __builtin_amdgcn_raw_buffer_store_b64(ov, rs, int((row * HD + 16 * n + 4 * lq) * 2u), 0, 0);
-        }
-        const float lse = lsum > 0.f ? m_run[nt] + __builtin_amdgcn_logf(lsum) : -INFINITY;
-        if (lq == 0) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, lse), rs, int(lse0 + row * 4u), 0, 0);
-      }
-    }
-    if (__any(ovf) && lane == 0) flag_status(p.status, PKV_STATUS_PARTIAL_RANGE);
-    return;
-  }
-
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int row = row0 + li + 16 * nt;
-    const float lsum = l_run[nt][0];
-    if (row < p.R) {
-      const int j = row / p.g;
-      const int hq = row - j * p.g;
-      const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-      uint16_t* dst = p.out + b * p.o_sb + j * p.o_ss + (h * p.g + hq) * p.o_sh + 4 * lq;
-#pragma unroll
-      for (int n = 0; n < DPL; ++n) {
-        const u32x2 ov = {pack_bf16x2(acc[nt][n][0] * inv, acc[nt][n][1] * inv),
-                          pack_bf16x2(acc[nt][n][2] * inv, acc[nt][n][3] * inv)};
-        *reinterpret_cast<u32x2*>(dst + 16 * n) = ov;
-      }
-    }
-  }
-}
+#include "pkv_prefill.h"
 
 // ---------------------------------------------------------------------------------------------
 // Host side
@@ -3490,25 +3056,10 @@ static void launch_decode_hd(const AttnParams& p, int batch, hipStream_t stream)
 constexpr int kPrefillNT = 2;
 constexpr int kPrefillW = 4;
 
-#ifndef PKV_PREFILL_LDS_NT
-#define PKV_PREFILL_LDS_NT 2
-#endif
-#ifndef PKV_PREFILL_LDS_W
-#define PKV_PREFILL_LDS_W 4
-#endif
-#ifndef PKV_PREFILL_LDS_NBUF
-#define PKV_PREFILL_LDS_NBUF 4  // 64 KiB of LDS per workgroup, one barrier per tile
-#endif
-
-#ifndef PKV_PREFILL_LDS_SUB
-#define PKV_PREFILL_LDS_SUB 1
-#endif
-
-static void launch_prefill_lds(const AttnParams& p, int batch, hipStream_t stream) {
-  constexpr int NT = PKV_PREFILL_LDS_NT, W = PKV_PREFILL_LDS_W;
-  constexpr int rows_per_wg = 16 * NT * W;
-  dim3 grid((p.R + rows_per_wg - 1) / rows_per_wg, p.n_kv, batch);
-  prefill_lds_kernel<NT, W, PKV_PREFILL_LDS_NBUF, PKV_PREFILL_LDS_SUB><<<grid, 64 * W, 0, stream>>>(p);
+template <int HD>
+static void launch_prefill_tiles(const AttnParams& p, int batch, hipStream_t stream) {
+  dim3 grid((p.R + pf::kRows - 1) / pf::kRows, p.n_kv, batch);
+  prefill_tile_kernel<HD, pf::kDirect><<<grid, 64 * pf::kWaves, 0, stream>>>(p);
 }
 
 template <int HD>
@@ -3883,9 +3434,8 @@ extern "C" int pkv_cascade_attn(const void* q, int64_t q_sb, int64_t q_ss, int64
   p.cascade_splits = S;
   if (!p.ws_cnt || !p.ws_o || !p.ws_ml) return fail(PKV_EINVAL, "%s: cascade launch without a workspace", fn);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  constexpr int NT = PKV_PREFILL_LDS_NT, W = PKV_PREFILL_LDS_W;
-  const dim3 pgrid((batch * R + 16 * NT * W - 1) / (16 * NT * W), rows::NKV, S);
-  prefill_lds_kernel<NT, W, PKV_PREFILL_LDS_NBUF, PKV_PREFILL_LDS_SUB, true><<<pgrid, 64 * W, 0, s>>>(p);
+  const dim3 pgrid((batch * R + pf::kRows - 1) / pf::kRows, rows::NKV, S);
+  prefill_tile_kernel<rows::HD, pf::kCascade><<<pgrid, 64 * pf::kWaves, 0, s>>>(p);
   launch_lean_g<Geom7B>(p, R, batch, grid, false, s);  // suffix pass + the merge of every part (two_pass)
   return check_launch(fn);
 }
@@ -3919,8 +3469,10 @@ extern "C" int pkv_prefill_attn(const void* q, int64_t q_sb, int64_t q_ss, int64
                        page_size, num_pages, max_blocks, status, s);
     if (rc) return rc;
   }
-  if (head_dim == 128 && page_size >= pf::TILE)
-    launch_prefill_lds(p, batch, s);
+  if (head_dim == 128 && page_size >= pf::Geo<128>::TOK)
+    launch_prefill_tiles<128>(p, batch, s);
+  else if (head_dim == 64 && page_size >= pf::Geo<64>::TOK)
+    launch_prefill_tiles<64>(p, batch, s);
   else if (head_dim == 128)
     launch_prefill_hd<128>(p, batch, s);
   else

@@ -1,0 +1,85 @@
+"""prefill_tile_kernel at the sizes where its pipeline, its rows and its pages can go wrong: every
+count of key stages around the ring depths (an odd count starts with an empty stage, the V ring holds
+4 and the K ring 5), row blocks with a remainder, rows that see no key, pages of exactly one stage,
+both head dims, with stale NaN behind every sequence.  Against the fp64 oracle at the bf16 tolerance."""
+import numpy as np
+import pytest
+import torch
+
+import prism_amd
+from oracle import paged_attention as pa
+from pkv_testutil import assert_attn_close, make_paged_case
+
+pytestmark = pytest.mark.gpu
+
+# head_dim, n_heads, n_kv, page, s_q, prefixes
+CASES = [
+    # 1 .. 12 stages of 32 tokens (head_dim 128), one sequence each
+    (128, 14, 2, 32, 19, [0, 14, 46, 77, 110, 141, 172, 206, 237, 269, 301, 333]),
+    # 1 .. 8 stages of 64 tokens (head_dim 64)
+    (64, 14, 2, 64, 19, [0, 46, 110, 173, 238, 301, 365, 429]),
+    # 128-row blocks: one row short, full, one row over, at a group size that does not divide them
+    (128, 5, 1, 256, 51, [3, 250]),
+    (64, 4, 4, 256, 128, [0, 64, 1]),
+    (64, 14, 2, 128, 37, [0, 63, 65, 1000]),
+    # pages smaller than a stage keep the per-wave kernel
+    (64, 14, 2, 32, 40, [0, 31, 100]),
+    (128, 8, 2, 16, 40, [0, 17, 100]),
+]
+
+
+def _nan_behind(d, ctx, s_q, page):
+    """Every slot past a sequence's keys in its last page holds NaN."""
+    for b, c in enumerate(ctx):
+        end = int(c) + s_q
+        last = int(d["block_table"][b, (end - 1) // page])
+        for cache in (d["k_cache"], d["v_cache"]):
+            cache[last, (end - 1) % page + 1:] = float("nan")
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("case", CASES, ids=[f"hd{c[0]}-p{c[3]}-s{c[4]}-g{c[1] // c[2]}" for c in CASES])
+def test_prefill_stage_and_row_edges(gpu, case, causal):
+    hd, nh, nk, page, s_q, ctx = case
+    cpu, d = make_paged_case(gpu, batch=len(ctx), ctx=ctx, page_size=page, n_kv=nk, n_heads=nh, head_dim=hd, s_q=s_q,
+                             seed=hd + page + s_q)
+    _nan_behind(d, ctx, s_q, page)
+    out = torch.full((len(ctx), s_q, nh, hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+    prism_amd.prefill_attention(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], cache_seqlens=d["cache_seqlens"],
+                                block_table=d["block_table"], causal=causal, out=out)
+    ref, _, _ = pa.flash_attn_with_kvcache_ref(cpu["q"], cpu["k_cache"], cpu["v_cache"], cpu["k"], cpu["v"],
+                                               cache_seqlens=cpu["cache_seqlens"], block_table=cpu["block_table"],
+                                               causal=causal)
+    torch.cuda.synchronize()
+    # rows that see a handful of keys: the output's own bf16 rounding passes 1e-2 where |o| > 2
+    few = np.array([[causal and c + j + 1 <= 8 for j in range(s_q)] for c in ctx])
+    got = out.float().cpu().numpy()
+    assert np.isfinite(got).all()
+    err = np.abs(got - ref)
+    ulp = np.maximum(1e-2, np.abs(ref) * 2.0 ** -7)
+    assert (err[few] <= ulp[few]).all() and err[~few].max(initial=0.0) <= 1e-2 and err.mean() <= 1e-3
+    assert prism_amd.read_status(gpu) == 0
+
+
+@pytest.mark.parametrize("hd,nh,nk", [(128, 14, 2), (64, 14, 2)])
+def test_prefill_rows_that_see_no_key(gpu, hd, nh, nk):
+    """Causal, no append, fewer cached keys than queries: the first rows see none and are zero."""
+    ctx, s_q = [5, 30, 100], 40
+    cpu, d = make_paged_case(gpu, batch=3, ctx=ctx, page_size=256, n_kv=nk, n_heads=nh, head_dim=hd, s_q=s_q, seed=3)
+    out = prism_amd.prefill_attention(d["q"], d["k_cache"], d["v_cache"], cache_seqlens=d["cache_seqlens"],
+                                      block_table=d["block_table"], causal=True)
+    ref, _, _ = pa.flash_attn_with_kvcache_ref(cpu["q"], cpu["k_cache"], cpu["v_cache"],
+                                               cache_seqlens=cpu["cache_seqlens"], block_table=cpu["block_table"],
+                                               causal=True)
+    torch.cuda.synchronize()
+    assert (out[0, :s_q - 5] == 0).all() and (out[1, :s_q - 30] == 0).all()
+    assert_attn_close(out[2:], ref[2:], "rows with keys")
+    assert np.isfinite(out.float().cpu().numpy()).all()
+
+
+def test_prefill_flags_a_bad_page(gpu):
+    cpu, d = make_paged_case(gpu, batch=2, ctx=[300, 10], page_size=64, n_kv=2, n_heads=14, head_dim=64, s_q=20, seed=9)
+    d["block_table"][0, 2] = 100000
+    prism_amd.prefill_attention(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], cache_seqlens=d["cache_seqlens"],
+                                block_table=d["block_table"], causal=True)
+    assert prism_amd.read_status(gpu) & 1
