@@ -256,6 +256,30 @@ int pkv_prefill_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
                      int32_t* status, void* stream);
 
 /*
+ * pkv_prefill_attn with a workspace for split keys: a call whose row blocks (128 rows of s_q *
+ * n_heads / n_kv, per KV head and sequence) would leave most of the card idle, such as a short turn
+ * onto a long cached prefix, cuts every block's keys into ranges, keeps each range's unnormalised
+ * output, row maximum and row sum in fp32 there and merges them in a second launch.  Same results
+ * up to the order of fp32 sums.  pkv_prefill_workspace_bytes() is what such a call needs, 0 where
+ * the keys are not split; workspace NULL never splits.  The same rules as pkv_decode_attn's
+ * workspace (the two may share one: the leading 64 KiB of counters are not touched).
+ */
+size_t pkv_prefill_workspace_bytes(int32_t batch, int32_t s_q, int32_t n_heads, int32_t n_kv,
+                                   int32_t head_dim, int32_t page_size, int32_t max_blocks);
+
+int pkv_prefill_attn_ws(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
+                        const void* k_new, int64_t kn_sb, int64_t kn_ss, int64_t kn_sh,
+                        const void* v_new, int64_t vn_sb, int64_t vn_ss, int64_t vn_sh,
+                        void* k_cache, void* v_cache, int64_t cache_page_stride,
+                        const int32_t* block_table, int64_t bt_stride, const int32_t* cache_seqlens,
+                        void* out, int64_t o_sb, int64_t o_ss, int64_t o_sh,
+                        void* workspace, size_t workspace_bytes,
+                        int32_t batch, int32_t s_q, int32_t n_heads, int32_t n_kv, int32_t head_dim,
+                        int32_t page_size, int32_t num_pages, int32_t max_blocks,
+                        int32_t causal, float softmax_scale,
+                        int32_t* status, void* stream);
+
+/*
  * Batched page copy (generalises engine/kv_cache.py:189-207, the per-layer, per-page copy_
  * loop of transfer_sequence; also copy-on-write of a shared partially filled page and
  * live-page migration).  For every tensor i < n_tensors and pair p < n_pages:

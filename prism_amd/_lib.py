@@ -98,6 +98,20 @@ _SIGNATURES = {
         _I32, c_float,
         _P, _P,
     ]),
+    "pkv_prefill_workspace_bytes": (c_size_t, [_I32] * 7),
+    "pkv_prefill_attn_ws": (c_int32, [
+        _P, _I64, _I64, _I64,
+        _P, _I64, _I64, _I64,
+        _P, _I64, _I64, _I64,
+        _P, _P, _I64,
+        _P, _I64, _P,
+        _P, _I64, _I64, _I64,
+        _P, c_size_t,                    # workspace
+        _I32, _I32, _I32, _I32, _I32,
+        _I32, _I32, _I32,
+        _I32, c_float,
+        _P, _P,
+    ]),
     "pkv_copy_pages": (c_int32, [
         _P, _P, _I32,                    # src_bases, dst_bases, n_tensors
         _P, _P, _P, _I32,                # src_ids, dst_ids, fill_slots, n_pages

@@ -23,6 +23,7 @@ needs).
 """
 from __future__ import annotations
 
+import functools
 import math
 import threading
 
@@ -187,6 +188,12 @@ def read_status(device: torch.device | str = "cuda", clear: bool = True) -> int:
         t.zero_()
         _recover(idx, v)
     return v
+
+
+@functools.lru_cache(maxsize=1024)
+def _prefill_bytes(*sizes: int) -> int:
+    """pkv_prefill_workspace_bytes, a function of the sizes alone."""
+    return _lib.load().pkv_prefill_workspace_bytes(*sizes)
 
 
 def _workspace(device: torch.device, nbytes: int, stream: int, allow_static: bool = False) -> torch.Tensor | None:
@@ -512,14 +519,18 @@ def flash_attn_with_kvcache(
             st.data_ptr(), stream)
         _lib.check(rc, "pkv_decode_attn")
     else:
-        rc = lib.pkv_prefill_attn(
+        # noalloc, or a capture without a sized workspace: the keys are not split
+        nbytes = 0 if noalloc else _prefill_bytes(batch, s_q, n_heads, n_kv, hd, page_size, max_blocks)
+        ws = _workspace(device, nbytes, stream, allow_static=True) if nbytes else None
+        rc = lib.pkv_prefill_attn_ws(
             q.data_ptr(), *qs, kp, *ks, vp, *vs,
             k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
             block_table.data_ptr(), block_table.stride(0), cache_seqlens.data_ptr(),
             out.data_ptr(), *os_,
+            ws.data_ptr() if ws is not None else 0, ws.numel() if ws is not None else 0,
             batch, s_q, n_heads, n_kv, hd, page_size, num_pages, max_blocks,
             1 if causal else 0, scale, st.data_ptr(), stream)
-        _lib.check(rc, "pkv_prefill_attn")
+        _lib.check(rc, "pkv_prefill_attn_ws")
     return out
 
 
@@ -620,11 +631,16 @@ def prefill_attention(q, k_cache, v_cache, k=None, v=None, *, cache_seqlens, blo
         return out
     st = status if status is not None else status_tensor(k_cache.device)
     scale = float(softmax_scale) if softmax_scale is not None else 1.0 / math.sqrt(hd)
-    rc = _lib.load().pkv_prefill_attn(
+    lib = _lib.load()
+    stream = _stream_ptr(q.device)
+    nbytes = _prefill_bytes(batch, s_q, n_heads, n_kv, hd, page_size, block_table.shape[1])
+    ws = _workspace(k_cache.device, nbytes, stream, allow_static=True)
+    rc = lib.pkv_prefill_attn_ws(
         q.data_ptr(), *qs, kp, *ks, vp, *vs,
         k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
         block_table.data_ptr(), block_table.stride(0), cache_seqlens.data_ptr(),
-        out.data_ptr(), *os_, batch, s_q, n_heads, n_kv, hd, page_size, num_pages,
-        block_table.shape[1], 1 if causal else 0, scale, st.data_ptr(), _stream_ptr(q.device))
-    _lib.check(rc, "pkv_prefill_attn")
+        out.data_ptr(), *os_, ws.data_ptr() if ws is not None else 0, ws.numel() if ws is not None else 0,
+        batch, s_q, n_heads, n_kv, hd, page_size, num_pages,
+        block_table.shape[1], 1 if causal else 0, scale, st.data_ptr(), stream)
+    _lib.check(rc, "pkv_prefill_attn_ws")
     return out

@@ -144,9 +144,8 @@ __device__ __forceinline__ void seq_lengths(const AttnParams& p, int b, int& c, 
 // length (ties by index), row blocks in descending order, KV heads innermost: longest-first list
 // scheduling, which shortens the launch's tail when prefixes differ (14B chunks onto prefixes
 // U{0..4096}: 242 -> 211 tile-times in a 512-slot model).  Batches above 64 keep launch order.
-__device__ __forceinline__ void prefill_item(const AttnParams& p, int& b, int& h, int& xblk) {
-  const int nx = int(gridDim.x), nkv = int(gridDim.y);
-  const int i = int(blockIdx.x) + nx * (int(blockIdx.y) + nkv * int(blockIdx.z));
+__device__ __forceinline__ void prefill_item(const AttnParams& p, int i, int nx, int& b, int& h, int& xblk) {
+  const int nkv = int(gridDim.y);
   const int per_seq = nx * nkv;
   const int rank = i / per_seq;
   const int r = i - rank * per_seq;
@@ -2586,7 +2585,7 @@ __global__ __launch_bounds__(64 * W) void prefill_kernel(const AttnParams p) {
   const int li = lane & 15;
   const int lq = lane >> 4;
   int b, h, xblk;
-  prefill_item(p, b, h, xblk);
+  prefill_item(p, int(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z)), int(gridDim.x), b, h, xblk);
 
   int c, L;
   seq_lengths(p, b, c, L);
@@ -3056,10 +3055,35 @@ static void launch_decode_hd(const AttnParams& p, int batch, hipStream_t stream)
 constexpr int kPrefillNT = 2;
 constexpr int kPrefillW = 4;
 
+// Key ranges per item of a prefill launch: as many as keep the workgroups within one round of two per
+// CU, no more than the block table has ranges of kMinStages for.  1 where the row blocks fill half the
+// card by themselves, and where no sequence can hold kSplitStages: a workgroup alone on its CU takes
+// 0.5-0.6 us per stage, and the ranges add a second launch of about 4 us.
+static int prefill_splits(int batch, int64_t R, int n_kv, int head_dim, int page_size, int max_blocks) {
+  const int tok = head_dim == 128 ? pf::Geo<128>::TOK : pf::Geo<64>::TOK;
+  if (page_size < tok) return 1;
+  const int64_t items = (R + pf::kRows - 1) / pf::kRows * n_kv * batch;
+  const int64_t by_grid = 2 * int64_t(device_cu_count()) / items;
+  const int64_t by_keys = int64_t(max_blocks) * page_size / (tok * pf::kMinStages);
+  const int64_t s = by_grid < by_keys ? by_grid : by_keys;
+  return s < 2 || by_keys * pf::kMinStages < pf::kSplitStages ? 1 : int(s);
+}
+static size_t ws_bytes_prefill(int batch, int64_t R, int n_kv, int head_dim, int splits) {
+  if (splits < 2) return 0;
+  return kCounterBytes + size_t((R + pf::kRows - 1) / pf::kRows * n_kv * batch) * splits * pf::kRows *
+                             (head_dim + 2) * sizeof(float);
+}
+
+// splits > 1 needs ws_o / ws_ml.
 template <int HD>
 static void launch_prefill_tiles(const AttnParams& p, int batch, hipStream_t stream) {
-  dim3 grid((p.R + pf::kRows - 1) / pf::kRows, p.n_kv, batch);
-  prefill_tile_kernel<HD, pf::kDirect><<<grid, 64 * pf::kWaves, 0, stream>>>(p);
+  const int nx = (p.R + pf::kRows - 1) / pf::kRows;
+  if (p.max_splits > 1) {
+    prefill_tile_kernel<HD, pf::kSplit><<<dim3(nx * p.max_splits, p.n_kv, batch), 64 * pf::kWaves, 0, stream>>>(p);
+    prefill_merge_kernel<HD><<<dim3(nx * (pf::kRows * HD / 1024), p.n_kv, batch), 256, 0, stream>>>(p, nx);
+    return;
+  }
+  prefill_tile_kernel<HD, pf::kDirect><<<dim3(nx, p.n_kv, batch), 64 * pf::kWaves, 0, stream>>>(p);
 }
 
 template <int HD>
@@ -3440,14 +3464,25 @@ extern "C" int pkv_cascade_attn(const void* q, int64_t q_sb, int64_t q_ss, int64
   return check_launch(fn);
 }
 
-extern "C" int pkv_prefill_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh, const void* k_new,
-                                int64_t kn_sb, int64_t kn_ss, int64_t kn_sh, const void* v_new, int64_t vn_sb,
-                                int64_t vn_ss, int64_t vn_sh, void* k_cache, void* v_cache, int64_t cache_page_stride,
-                                const int32_t* block_table, int64_t bt_stride, const int32_t* cache_seqlens, void* out,
-                                int64_t o_sb, int64_t o_ss, int64_t o_sh, int32_t batch, int32_t s_q, int32_t n_heads,
-                                int32_t n_kv, int32_t head_dim, int32_t page_size, int32_t num_pages,
-                                int32_t max_blocks, int32_t causal, float softmax_scale, int32_t* status,
-                                void* stream) {
+extern "C" size_t pkv_prefill_workspace_bytes(int32_t batch, int32_t s_q, int32_t n_heads, int32_t n_kv,
+                                              int32_t head_dim, int32_t page_size, int32_t max_blocks) {
+  using namespace pkv;
+  if (batch <= 0 || s_q <= 0 || n_kv <= 0 || n_heads <= 0 || max_blocks <= 0 || page_size <= 0 ||
+      (head_dim != 64 && head_dim != 128))
+    return 0;
+  const int64_t R = int64_t(s_q) * (n_heads / n_kv);
+  return ws_bytes_prefill(batch, R, n_kv, head_dim, prefill_splits(batch, R, n_kv, head_dim, page_size, max_blocks));
+}
+
+extern "C" int pkv_prefill_attn_ws(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh, const void* k_new,
+                                   int64_t kn_sb, int64_t kn_ss, int64_t kn_sh, const void* v_new, int64_t vn_sb,
+                                   int64_t vn_ss, int64_t vn_sh, void* k_cache, void* v_cache,
+                                   int64_t cache_page_stride, const int32_t* block_table, int64_t bt_stride,
+                                   const int32_t* cache_seqlens, void* out, int64_t o_sb, int64_t o_ss, int64_t o_sh,
+                                   void* workspace, size_t workspace_bytes, int32_t batch, int32_t s_q,
+                                   int32_t n_heads, int32_t n_kv, int32_t head_dim, int32_t page_size,
+                                   int32_t num_pages, int32_t max_blocks, int32_t causal, float softmax_scale,
+                                   int32_t* status, void* stream) {
   using namespace pkv;
   clear_error();
   const char* fn = "pkv_prefill_attn";
@@ -3462,6 +3497,18 @@ extern "C" int pkv_prefill_attn(const void* q, int64_t q_sb, int64_t q_ss, int64
   fill_params(p, q, q_sb, q_ss, q_sh, k_new, kn_sb, kn_ss, kn_sh, v_new, vn_sb, vn_ss, vn_sh, k_cache, v_cache,
               cache_page_stride, block_table, bt_stride, cache_seqlens, out, o_sb, o_ss, o_sh, s_q, n_heads, n_kv,
               page_size, num_pages, max_blocks, causal, softmax_scale, status);
+  if (workspace) {
+    if (!aligned16(workspace)) return fail(PKV_EINVAL, "%s: workspace not 16-byte aligned", fn);
+    const int splits = prefill_splits(batch, R, n_kv, head_dim, page_size, max_blocks);
+    if (splits > 1) {
+      const size_t need = ws_bytes_prefill(batch, R, n_kv, head_dim, splits);
+      if (workspace_bytes < need)
+        return fail(PKV_ENOSPC, "%s: workspace %zu bytes < %zu needed", fn, workspace_bytes, need);
+      p.max_splits = splits;
+      p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
+      p.ws_ml = p.ws_o + size_t((R + pf::kRows - 1) / pf::kRows * n_kv * batch) * splits * pf::kRows * head_dim;
+    }
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (k_new) {
     rc = launch_append(fn, k_new, kn_sb, kn_ss, kn_sh, v_new, vn_sb, vn_ss, vn_sh, k_cache, v_cache,
@@ -3478,6 +3525,20 @@ extern "C" int pkv_prefill_attn(const void* q, int64_t q_sb, int64_t q_ss, int64
   else
     launch_prefill_hd<64>(p, batch, s);
   return check_launch(fn);
+}
+
+extern "C" int pkv_prefill_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh, const void* k_new,
+                                int64_t kn_sb, int64_t kn_ss, int64_t kn_sh, const void* v_new, int64_t vn_sb,
+                                int64_t vn_ss, int64_t vn_sh, void* k_cache, void* v_cache, int64_t cache_page_stride,
+                                const int32_t* block_table, int64_t bt_stride, const int32_t* cache_seqlens, void* out,
+                                int64_t o_sb, int64_t o_ss, int64_t o_sh, int32_t batch, int32_t s_q, int32_t n_heads,
+                                int32_t n_kv, int32_t head_dim, int32_t page_size, int32_t num_pages,
+                                int32_t max_blocks, int32_t causal, float softmax_scale, int32_t* status,
+                                void* stream) {
+  return pkv_prefill_attn_ws(q, q_sb, q_ss, q_sh, k_new, kn_sb, kn_ss, kn_sh, v_new, vn_sb, vn_ss, vn_sh, k_cache,
+                             v_cache, cache_page_stride, block_table, bt_stride, cache_seqlens, out, o_sb, o_ss, o_sh,
+                             nullptr, 0, batch, s_q, n_heads, n_kv, head_dim, page_size, num_pages, max_blocks,
+                             causal, softmax_scale, status, stream);
 }
 
 #ifdef PKV_TILE_STAMPS

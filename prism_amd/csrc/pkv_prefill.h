@@ -70,7 +70,32 @@ __device__ __forceinline__ float max2(float a, float b) { return __builtin_eleme
 enum Dest {
   kDirect,   // the bf16 output rows
   kCascade,  // the shared-prefix pass of a cascade launch: fp16 O / l and the log-sum-exp of one key split
+  kSplit,    // one of max_splits key ranges: fp32 O and (m, l) for prefill_merge_kernel
 };
+
+// Key ranges.  A call with few row blocks (150 tokens onto 3500 at the 7B shape: 36 workgroups of 115
+// stages) leaves most CUs idle at 0.6 us per stage; cut into 14 ranges each, it takes 30 us a call
+// instead of 70, the merge launch included.  The partials stay fp32.
+// Key ranges of an item of n stages in a kSplit launch: `chunk` stages each, at least kMinStages (a
+// range pays about two stages' time to start and one to end).  One range writes its rows directly.
+constexpr int kMinStages = 4;
+constexpr int kSplitStages = 16;  // stages a sequence must be able to hold for a kSplit launch
+struct Ranges {
+  int chunk, count;
+};
+__device__ __forceinline__ Ranges ranges_of(const AttnParams& p, int n) {
+  Ranges r;
+  r.chunk = max((n + p.max_splits - 1) / p.max_splits, kMinStages);
+  r.count = n > 0 ? (n + r.chunk - 1) / r.chunk : 1;
+  return r;
+}
+
+// Stages that rows up to blk_last of a sequence of L keys see.
+template <int TOK>
+__device__ __forceinline__ int stages_of(const AttnParams& p, int L, int blk_last) {
+  const int t_stop = p.causal ? min(L, L - p.s_q + blk_last / p.g + 1) : L;
+  return t_stop > 0 ? (t_stop + TOK - 1) / TOK : 0;
+}
 
 __device__ __forceinline__ u32x4 lds_read16(uint32_t addr) {
   return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(uintptr_t(addr));
@@ -127,6 +152,8 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
   const int R_all = CASCADE ? p.batch * p.R : p.R;  // query rows of the launch's row space
   int t_first = 0;                                  // first stage of this workgroup's key range
   int n;                                            // its stages
+  int split = 0;                                    // kSplit: which range of the item
+  bool whole = true;                                // kSplit: the item's only range
   if constexpr (CASCADE) {
     xblk = blockIdx.x;
     h = blockIdx.y;
@@ -134,7 +161,15 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     c = 0;
     L = p.k0;
   } else {
-    prefill_item(p, b, h, xblk);
+    const int i = int(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
+    if constexpr (DEST == pf::kSplit) {
+      // the ranges of an item are consecutive workgroups: with 8 or 16 of them each XCD's L2 serves
+      // the same keys for every row block
+      split = i % p.max_splits;
+      prefill_item(p, i / p.max_splits, int(gridDim.x) / p.max_splits, b, h, xblk);
+    } else {
+      prefill_item(p, i, int(gridDim.x), b, h, xblk);
+    }
     seq_lengths(p, b, c, L);
   }
   b = __builtin_amdgcn_readfirstlane(b);
@@ -161,8 +196,14 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     t_first = int(blockIdx.z) * chunk;
     n = max(min(chunk, n_shared - t_first), 0);
   } else {
-    const int t_stop = p.causal ? min(L, L - p.s_q + blk_last / p.g + 1) : L;
-    n = t_stop > 0 ? (t_stop + TOK - 1) / TOK : 0;
+    n = pf::stages_of<TOK>(p, L, blk_last);
+    if constexpr (DEST == pf::kSplit) {
+      const pf::Ranges r = pf::ranges_of(p, n);
+      if (split >= r.count) return;
+      whole = r.count == 1;
+      t_first = split * r.chunk;
+      n = min(r.chunk, n - t_first);
+    }
   }
 
   // Q rows (key step kk: elements 16 kk + 8 hi .. + 7 of row row0 + ln) and the row's last visible key
@@ -519,6 +560,23 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     if (__any(ovf) && lane == 0) flag_status(p.status, PKV_STATUS_PARTIAL_RANGE);
     return;
   }
+  if constexpr (DEST == pf::kSplit) {
+    if (!whole) {
+      if (lo.real) {
+        const int64_t wrow = (int64_t((b * p.n_kv + h) * (int(gridDim.x) / p.max_splits) + xblk) * p.max_splits + split) *
+                                 pf::kRows + lo.r - blk_row0;
+        float* dst = p.ws_o + wrow * HD + 4 * hi;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4*>(dst + 32 * dt + 8 * q) =
+                f32x4{o[dt][4 * q], o[dt][4 * q + 1], o[dt][4 * q + 2], o[dt][4 * q + 3]};
+        if (hi == 0) *reinterpret_cast<f32x2*>(p.ws_ml + 2 * wrow) = f32x2{m_run, lsum};
+      }
+      return;
+    }
+  }
   if (lo.real) {
     uint16_t* dst = p.out + lo.b * p.o_sb + lo.j * p.o_ss + lo.hq * p.o_sh + 4 * hi;
 #pragma unroll
@@ -530,4 +588,52 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
         *reinterpret_cast<u32x2*>(dst + 32 * dt + 8 * q) = ov;
       }
   }
+}
+
+// Merge of a kSplit launch: grid (row block x HD / 8, KV head, sequence), 1024 / HD rows of an item per
+// workgroup, one f32x4 of a row per thread.  Every range's load of a batch of 8 goes out before any is used.
+template <int HD>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p, int nx) {
+  constexpr int TPR = HD / 4, RPW = 256 / TPR, B = 8;
+  constexpr int BLOCKS = pf::kRows / RPW;  // workgroups per item
+  const int xblk = int(blockIdx.x) / BLOCKS, h = blockIdx.y, b = blockIdx.z;
+  const int r = (int(blockIdx.x) % BLOCKS) * RPW + int(threadIdx.x) / TPR;  // row in the block
+  const int blk_row0 = xblk * pf::kRows;
+  int c, L;
+  seq_lengths(p, b, c, L);
+  const int count = pf::ranges_of(p, pf::stages_of<pf::Geo<HD>::TOK>(p, L, min(blk_row0 + pf::kRows, p.R) - 1)).count;
+  const int row = blk_row0 + r;
+  if (count <= 1 || row >= p.R) return;
+  const int64_t w0 = int64_t((b * p.n_kv + h) * nx + xblk) * p.max_splits * pf::kRows + r;
+  const int d = (int(threadIdx.x) % TPR) * 4;
+  float m = -INFINITY, l = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < count; s0 += B) {
+    f32x4 po[B];
+    f32x2 pm[B];
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+      const int64_t w = w0 + int64_t(min(s0 + k, count - 1)) * pf::kRows;
+      po[k] = *reinterpret_cast<const f32x4*>(p.ws_o + w * HD + d);
+      pm[k] = *reinterpret_cast<const f32x2*>(p.ws_ml + 2 * w);
+    }
+    float m_new = m;
+#pragma unroll
+    for (int k = 0; k < B; ++k) m_new = fmaxf(m_new, pm[k][0]);
+    const float keep = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);
+    l *= keep;
+    o *= keep;
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+      // a range of which the row sees no key has l = 0 and m = -inf
+      const float wt = s0 + k < count && pm[k][1] > 0.f ? fast_exp2(pm[k][0] - m_new) : 0.f;
+      l += wt * pm[k][1];
+      o += wt * po[k];
+    }
+    m = m_new;
+  }
+  const int j = row / p.g;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  uint16_t* dst = p.out + b * p.o_sb + j * p.o_ss + (h * p.g + row - j * p.g) * p.o_sh + d;
+  *reinterpret_cast<u32x2*>(dst) = u32x2{pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv)};
 }

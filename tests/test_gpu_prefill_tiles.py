@@ -83,3 +83,61 @@ def test_prefill_flags_a_bad_page(gpu):
     prism_amd.prefill_attention(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], cache_seqlens=d["cache_seqlens"],
                                 block_table=d["block_table"], causal=True)
     assert prism_amd.read_status(gpu) & 1
+
+
+# head_dim, n_heads, n_kv, page, s_q, prefixes: few enough row blocks that the keys split, over ranges
+# of one, a few and the most stages, uneven lengths (some sequences one range, some none)
+SPLIT_CASES = [
+    (128, 28, 4, 256, 33, [3000]),
+    (128, 8, 8, 64, 129, [0, 700, 5]),
+    (64, 14, 2, 256, 70, [5000, 0]),
+    (64, 2, 2, 64, 257, [1, 1500, 255]),
+    (128, 7, 1, 256, 20, [16000]),
+]
+
+
+@pytest.mark.parametrize("append", [True, False])
+@pytest.mark.parametrize("case", SPLIT_CASES, ids=[f"hd{c[0]}-kv{c[2]}-s{c[4]}" for c in SPLIT_CASES])
+def test_prefill_split_keys_matches_unsplit_and_oracle(gpu, case, append):
+    hd, nh, nk, page, s_q, ctx = case
+    cpu, d = make_paged_case(gpu, batch=len(ctx), ctx=ctx, page_size=page, n_kv=nk, n_heads=nh, head_dim=hd, s_q=s_q,
+                             seed=hd + nk + s_q)
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True)
+    k, v = (d["k"], d["v"]) if append else (None, None)
+    assert prism_amd._lib.load().pkv_prefill_workspace_bytes(len(ctx), s_q, nh, nk, hd, page,
+                                                             d["block_table"].shape[1]) > 0
+    out = torch.full((len(ctx), s_q, nh, hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+    one = torch.full_like(out, float("nan"))
+    prism_amd.prefill_attention(d["q"], d["k_cache"], d["v_cache"], k, v, out=out, **kw)
+    prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], k, v, out=one, noalloc=True, **kw)
+    ref, _, _ = pa.flash_attn_with_kvcache_ref(cpu["q"], cpu["k_cache"], cpu["v_cache"], cpu["k"] if append else None,
+                                               cpu["v"] if append else None, cache_seqlens=cpu["cache_seqlens"],
+                                               block_table=cpu["block_table"], causal=True)
+    torch.cuda.synchronize()
+    a, b = out.float().cpu().numpy(), one.float().cpu().numpy()
+    assert np.isfinite(a).all() and np.isfinite(b).all()
+    # the same products in another order of fp32 sums (and another running max per range, so P rounds
+    # differently): two bf16 units of the row, or of 1e-2
+    assert (np.abs(a - b) <= np.maximum(1e-2, np.abs(b) * 2.0 ** -6)).all()
+    few = np.array([[c + j + (1 if append else 1 - s_q) <= 8 for j in range(s_q)] for c in ctx])
+    err = np.abs(a - ref)
+    assert err[~few].max(initial=0.0) <= 1e-2 and err.mean() <= 1e-3
+    assert prism_amd.read_status(gpu) == 0
+
+
+def test_prefill_captured_without_a_workspace_runs_unsplit(gpu):
+    """A capture sizes no workspace of its own: the captured call and its replays give the eager
+    unsplit result."""
+    cpu, d = make_paged_case(gpu, batch=1, ctx=[900], page_size=256, n_kv=4, n_heads=28, head_dim=128, s_q=40, seed=1)
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, noalloc=True)
+    want = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], **kw)
+    out = torch.empty_like(want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], out=out, **kw)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
