@@ -3074,13 +3074,50 @@ static size_t ws_bytes_prefill(int batch, int64_t R, int n_kv, int head_dim, int
                              (head_dim + 2) * sizeof(float);
 }
 
+// Speculative verify on prefill_tile_kernel's two-wave form.  decode_lean_kernel's verify rows are one
+// serial chain per wave at one wave per SIMD, with a 1.8-2.4 us segment start per sequence and a
+// 7-8 us merge launch; this form runs six waves per CU and starts a range in about 2.5 us.  Per call,
+// lean / tiles: 7B B = 8 26.4 / 20.1 us, B = 32 42.5 / 39.7, B = 64 over a shared 2048-token prefix
+// 57.8 / 50.2, 14B B = 16 42.4 / 41.8, one TP-4 shard B = 16 32.2 / 19.7, 0.5B B = 64 40.0 / 27.1; ahead
+// or level at each of 34 random draws up to one (sequence, KV head) per CU.  Past that the ranges no
+// longer fit one round: 7B B = 128 58.4 / 64.1, so the rule ends there.
+// It takes the calls decode_lean_kernel would take
+// with more than 16 query rows per KV head (both round P to bf16 once), unless a flag asks for a merge
+// or a grid.  Key ranges per KV head: about one round of kVerifyPerCu workgroups per CU over all heads.
+constexpr size_t kScratchBytes = size_t(48) << 20;  // pkv_decode_attn_noalloc's static scratch
+static int verify_target(int n_kv) {
+  const int t = pf::kVerifyPerCu * device_cu_count() / n_kv;
+  return t > 0 ? t : 1;
+}
+// ceil(total / chunk) ranges and at most one more per sequence
+static int64_t verify_slots(int batch, int n_kv) { return (int64_t(verify_target(n_kv)) + batch) * n_kv; }
+static size_t ws_bytes_verify(int batch, int n_kv, int head_dim) {
+  return kCounterBytes + size_t(verify_slots(batch, n_kv)) * pf::kVerifyRows * (head_dim + 2) * sizeof(float) +
+         size_t(batch) * 2 * sizeof(int32_t);
+}
+// Only where the ranges fit the static scratch, so that a call takes the same kernel with and without
+// a workspace of its own.
+static bool use_verify_tiles(int batch, int n_kv, int head_dim, int R, int page_size, bool lean, int32_t flags) {
+  return lean && R > 16 && page_size >= (head_dim == 128 ? pf::Geo<128>::TOK : pf::Geo<64>::TOK) &&
+         (flags & ~PKV_DECODE_RESET_COUNTERS) == 0 && int64_t(batch) * n_kv <= device_cu_count() &&
+         ws_bytes_verify(batch, n_kv, head_dim) <= kScratchBytes;
+}
+template <int HD>
+static void launch_verify_tiles(const AttnParams& p, int batch, hipStream_t stream) {
+  prefill_tile_kernel<HD, pf::kSplit, pf::kVerifyWaves>
+      <<<unsigned(verify_slots(batch, p.n_kv)), 64 * pf::kVerifyWaves, 0, stream>>>(p);
+  prefill_merge_kernel<HD, pf::kVerifyRows>
+      <<<dim3((p.R * HD + 1023) / 1024, p.n_kv, batch), 256, 0, stream>>>(p, 1);
+}
+
 // splits > 1 needs ws_o / ws_ml.
 template <int HD>
 static void launch_prefill_tiles(const AttnParams& p, int batch, hipStream_t stream) {
   const int nx = (p.R + pf::kRows - 1) / pf::kRows;
   if (p.max_splits > 1) {
     prefill_tile_kernel<HD, pf::kSplit><<<dim3(nx * p.max_splits, p.n_kv, batch), 64 * pf::kWaves, 0, stream>>>(p);
-    prefill_merge_kernel<HD><<<dim3(nx * (pf::kRows * HD / 1024), p.n_kv, batch), 256, 0, stream>>>(p, nx);
+    prefill_merge_kernel<HD, pf::kRows>
+        <<<dim3(nx * (pf::kRows * HD / 1024), p.n_kv, batch), 256, 0, stream>>>(p, nx);
     return;
   }
   prefill_tile_kernel<HD, pf::kDirect><<<dim3(nx, p.n_kv, batch), 64 * pf::kWaves, 0, stream>>>(p);
@@ -3109,6 +3146,10 @@ extern "C" size_t pkv_decode_workspace_bytes(int32_t batch, int32_t s_q, int32_t
   if (use_lean_kernel(batch, head_dim, n_kv, R, page_size, split_tokens, 0)) {
     const size_t lean = ws_bytes_lean(lean_grid(0), R);
     need = lean > need ? lean : need;
+    if (use_verify_tiles(batch, n_kv, head_dim, R, page_size, true, 0)) {
+      const size_t v = ws_bytes_verify(batch, n_kv, head_dim);
+      need = v > need ? v : need;
+    }
   }
   return need;
 }
@@ -3124,7 +3165,6 @@ namespace pkv {
 // device current, and is kept per device.  Every call on a GPU shares that GPU's array, so calls
 // that overlap on one GPU (different streams, no ordering between them) race.
 // ---------------------------------------------------------------------------------------------
-constexpr size_t kScratchBytes = size_t(48) << 20;
 static __device__ __align__(256) char scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
@@ -3210,7 +3250,15 @@ static int decode_attn(const char* fn, bool use_scratch, const void* q, int64_t 
   if (batch == 0) return PKV_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int grid = lean ? lean_grid(flags) : 0;
-  const size_t need = lean ? ws_bytes_lean(grid, R) : (ms > 1 ? ws_bytes(batch, R, n_kv, head_dim, ms) : 0);
+  // The two-wave form reads the new rows back in the launch that stores them, so a head's row must
+  // not share a 128-byte cache line with another head's or token's, which another workgroup of the CU
+  // may have read before the store.
+  const bool lines = ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) |
+                       uintptr_t(cache_page_stride) * 2) & 127) == 0;
+  const bool verify = (lines || !k_new) && use_verify_tiles(batch, n_kv, head_dim, R, page_size, lean, flags);
+  const size_t need = verify ? ws_bytes_verify(batch, n_kv, head_dim)
+                      : lean ? ws_bytes_lean(grid, R)
+                             : (ms > 1 ? ws_bytes(batch, R, n_kv, head_dim, ms) : 0);
   if (lean && need - kCounterBytes >= (size_t(1) << 31))
     return fail(PKV_EINVAL, "%s: %d workgroups need a %zu-byte workspace (partials must stay under 2 GiB)",
                 fn, grid, need);
@@ -3249,6 +3297,17 @@ static int decode_attn(const char* fn, bool use_scratch, const void* q, int64_t 
   p.rot_cos = static_cast<const uint16_t*>(rot_cos);
   p.rot_sin = static_cast<const uint16_t*>(rot_sin);
   p.n_pos = n_pos;
+  if (verify) {
+    p.lean_grid = verify_target(n_kv);
+    p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
+    p.ws_ml = p.ws_o + size_t(verify_slots(batch, n_kv)) * pf::kVerifyRows * head_dim;
+    p.ws_cnt = reinterpret_cast<int32_t*>(p.ws_ml + size_t(verify_slots(batch, n_kv)) * pf::kVerifyRows * 2);
+    if (head_dim == 128)
+      launch_verify_tiles<128>(p, batch, s);
+    else
+      launch_verify_tiles<64>(p, batch, s);
+    return check_launch(fn);
+  }
   if (lean) {
     p.ws_cnt = static_cast<int32_t*>(workspace);
     p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);

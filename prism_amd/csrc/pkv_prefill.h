@@ -54,13 +54,17 @@ struct Geo {
 
 constexpr int kWaves = 4;
 constexpr int kRows = 32 * kWaves;   // query rows per workgroup
-constexpr int kRingK = 5, kRingV = 4;
+// Verify's workgroups: two waves, 64 query rows.  Their copies run one stage less ahead, so that three
+// workgroups' rings fit a CU's LDS.
+constexpr int kVerifyWaves = 2;
+constexpr int kVerifyRows = 32 * kVerifyWaves;
+constexpr int kVerifyPerCu = 3;
 
-// At most n of this wave's copies may stay in flight.
-template <int N>
+// At most N of this wave's copies may stay in flight (LGKM: and none of its LDS reads).
+template <int N, bool LGKM = false>
 __device__ __forceinline__ void wait_vm() {
-  static_assert(N <= 15, "vmcnt immediate");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | N);
+  static_assert(N < 64, "vmcnt immediate");
+  __builtin_amdgcn_s_waitcnt((LGKM ? 0x0070 : 0x0F70) | (N & 15) | ((N >> 4) << 14));
 }
 
 // The larger of the lane's scores (never NaN unless the inputs are, and then the row is NaN anyway).
@@ -79,6 +83,7 @@ enum Dest {
 // Key ranges of an item of n stages in a kSplit launch: `chunk` stages each, at least kMinStages (a
 // range pays about two stages' time to start and one to end).  One range writes its rows directly.
 constexpr int kMinStages = 4;
+constexpr int kMinVerifyStages = 5;
 constexpr int kSplitStages = 16;  // stages a sequence must be able to hold for a kSplit launch
 struct Ranges {
   int chunk, count;
@@ -130,18 +135,80 @@ __device__ __forceinline__ float max_halves(float v) {
 __device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
 
+// Verify's ranges.  The stages of all sequences, sequence after sequence, are cut into ranges of one
+// length (`chunk`: about lean_grid ranges for each KV head, at least kMinVerifyStages stages each: 2 cost
+// the TP-4 shard 12 us, 4 to 6 are level), each inside
+// one sequence: a ragged batch keeps every workgroup at the same work, whatever the longest sequence.
+// Range w of KV head h is workgroup w n_kv + h, so that each XCD's L2 serves few heads (a cached prefix
+// that the batch shares is then read once per XCD and head).
+constexpr int kVerifyBatch = 256;
+struct VerifyPlan {
+  int n[kVerifyBatch / 64];  // stages of sequence 64 i + lane (0 past the batch)
+  int chunk;
+};
+template <int TOK>
+__device__ __forceinline__ VerifyPlan verify_plan(const AttnParams& p) {
+  const int lane = threadIdx.x & 63;
+  const int cap = p.max_blocks << p.log2_page;
+  VerifyPlan v;
+#pragma unroll
+  for (int i = 0; i < kVerifyBatch / 64; ++i) {
+    v.n[i] = 0;
+    if (64 * i < p.batch && 64 * i + lane < p.batch) {
+      const int c = min(max(p.seqlens[64 * i + lane], 0), cap);  // as seq_lengths clamps it
+      v.n[i] = max(stages_of<TOK>(p, min(c + (p.has_new ? p.s_q : 0), cap), p.R - 1), 1);
+    }
+  }
+  int total = 0;
+#pragma unroll
+  for (int i = 0; i < kVerifyBatch / 64; ++i)
+    if (64 * i < p.batch) total += __builtin_amdgcn_readlane(wave_incl_scan(v.n[i]), 63);
+  v.chunk = max((total + p.lean_grid - 1) / p.lean_grid, kMinVerifyStages);
+  // every sequence's last range may be short: lengthen the ranges until they fit one round
+  for (int tries = 0; tries < 16; ++tries) {
+    int ranges = 0;
+#pragma unroll
+    for (int i = 0; i < kVerifyBatch / 64; ++i)
+      if (64 * i < p.batch) ranges += __builtin_amdgcn_readlane(wave_incl_scan((v.n[i] + v.chunk - 1) / v.chunk), 63);
+    if (ranges <= max(p.lean_grid, p.batch)) break;
+    v.chunk += max(v.chunk / 16, 1);
+  }
+  return v;
+}
+// Calls f(i, ranges of sequence 64 i + lane, their inclusive sum inside the 64, ranges before the 64).
+template <typename F>
+__device__ __forceinline__ void verify_ranges(const AttnParams& p, const VerifyPlan& v, F&& f) {
+  int base = 0;
+#pragma unroll
+  for (int i = 0; i < kVerifyBatch / 64; ++i) {
+    if (64 * i < p.batch) {
+      const int r = (v.n[i] + v.chunk - 1) / v.chunk;
+      const int incl = wave_incl_scan(r);
+      f(i, r, incl, base);
+      base += __builtin_amdgcn_readlane(incl, 63);
+    }
+  }
+}
+
 }  // namespace pf
 
 // CASCADE form (DEST == kCascade): grid (row blocks of the whole batch's query rows, KV heads, key
 // splits); block-table row 0 holds the shared pages; split z covers stages [z chunk, (z + 1) chunk)
 // of the k0 shared keys, which every row sees whole; the result is a partial (fp16 O / l and fp32
 // log-sum-exp) in workspace slot 2 G + b S + z of each row.
-template <int HD, int DEST>
-__global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const AttnParams p) {
+//
+// W waves own 32 W rows.  W = 2 (kSplit only) is speculative verify: one row block per (sequence, KV
+// head); each range appends the new rows it covers itself, before it copies them.
+template <int HD, int DEST, int W = pf::kWaves>
+__global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParams p) {
   using G = pf::Geo<HD>;
+  constexpr int kRows = 32 * W;
+  constexpr int kLead = W == pf::kWaves ? 3 : 2;  // iterations between a copy's issue and its use
+  constexpr int kRing = kLead + 1;                // slots of the K and of the V ring
+  constexpr int kCopies = 8 / W;                  // copies of a K (or V) stage per wave
   constexpr int TT = G::TT, DT = G::DT, KK = G::KK, TOK = G::TOK;
   constexpr bool CASCADE = DEST == pf::kCascade;
-  __shared__ __attribute__((aligned(16))) char lds[(pf::kRingK + pf::kRingV) * G::STAGE];
+  __shared__ __attribute__((aligned(16))) char lds[2 * kRing * G::STAGE];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -152,8 +219,7 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
   const int R_all = CASCADE ? p.batch * p.R : p.R;  // query rows of the launch's row space
   int t_first = 0;                                  // first stage of this workgroup's key range
   int n;                                            // its stages
-  int split = 0;                                    // kSplit: which range of the item
-  bool whole = true;                                // kSplit: the item's only range
+  int split = 0, count = 1, chunk = 0;              // kSplit: which range of the item, of how many, stages each
   if constexpr (CASCADE) {
     xblk = blockIdx.x;
     h = blockIdx.y;
@@ -162,13 +228,38 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     L = p.k0;
   } else {
     const int i = int(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));
-    if constexpr (DEST == pf::kSplit) {
+    if constexpr (W != pf::kWaves) {
+      // found below
+    } else if constexpr (DEST == pf::kSplit) {
       // the ranges of an item are consecutive workgroups: with 8 or 16 of them each XCD's L2 serves
       // the same keys for every row block
       split = i % p.max_splits;
       prefill_item(p, i / p.max_splits, int(gridDim.x) / p.max_splits, b, h, xblk);
     } else {
       prefill_item(p, i, int(gridDim.x), b, h, xblk);
+    }
+    if constexpr (W != pf::kWaves) {
+      xblk = 0;
+      h = i % p.n_kv;
+      const int w = i / p.n_kv;
+      const pf::VerifyPlan v = pf::verify_plan<TOK>(p);
+      chunk = v.chunk;
+      b = -1;
+      pf::verify_ranges(p, v, [&](int k, int r, int incl, int base) {
+        const uint64_t hit = __ballot(base + incl > w);
+        if (b < 0 && hit) {
+          const int first = int(__builtin_ctzll(hit));
+          b = 64 * k + first;
+          count = __builtin_amdgcn_readlane(r, first);
+          split = w - base - (__builtin_amdgcn_readlane(incl, first) - count);
+        }
+      });
+      if (b < 0) return;  // fewer ranges than the grid allows for
+      // for the merge: where the sequence's ranges start, and how many they are
+      if (h == 0 && split == 0 && threadIdx.x == 0) {
+        p.ws_cnt[2 * b] = w;
+        p.ws_cnt[2 * b + 1] = count;
+      }
     }
     seq_lengths(p, b, c, L);
   }
@@ -184,11 +275,11 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
   sv.t_end = L;
   sv.bt = p.block_table + int64_t(b) * p.bt_stride;
 
-  const int blk_row0 = xblk * pf::kRows;
+  const int blk_row0 = xblk * kRows;
   if (blk_row0 >= R_all) return;
   const int row0 = blk_row0 + wave * 32;
   // the block's last row sees the most keys (rows increase with j)
-  const int blk_last = min(blk_row0 + pf::kRows, R_all) - 1;
+  const int blk_last = min(blk_row0 + kRows, R_all) - 1;
   if constexpr (CASCADE) {
     if (blockIdx.z == 0 && h == 0) cascade_check_sharing(p, blk_row0 / p.R, blk_last / p.R);
     const int n_shared = p.k0 / TOK;
@@ -198,11 +289,24 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
   } else {
     n = pf::stages_of<TOK>(p, L, blk_last);
     if constexpr (DEST == pf::kSplit) {
-      const pf::Ranges r = pf::ranges_of(p, n);
-      if (split >= r.count) return;
-      whole = r.count == 1;
-      t_first = split * r.chunk;
-      n = min(r.chunk, n - t_first);
+      if constexpr (W == pf::kWaves) {
+        const pf::Ranges r = pf::ranges_of(p, n);
+        if (split >= r.count) return;
+        count = r.count;
+        chunk = r.chunk;
+      }
+      t_first = split * chunk;
+      n = min(chunk, n - t_first);
+    }
+  }
+
+  if constexpr (W != pf::kWaves) {
+    // the new rows among this range's keys: stored to the cache, then copied from there like any other
+    const int a0 = max(c, t_first * TOK), a1 = min(L, (t_first + n) * TOK);
+    if (p.has_new && a0 < a1) {
+      append_rows<HD>(p, sv, a0, a1, int(threadIdx.x), 64 * W);
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): acknowledged, also of the other wave after the barrier
+      raw_barrier();
     }
   }
 
@@ -247,12 +351,13 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
 
   // ---- tile copies ----
   // Copy i (< 8) of a K or V stage: rows RPC i .. + RPC - 1, lane l -> row + l / CPR, LDS chunk l %
-  // CPR <- global chunk (l % CPR) ^ swizzle(row).  Wave w issues copies w and w + 4, which share the
-  // swizzle, so each lane's offset inside a stage's buffer is one register and i a scalar offset.
+  // CPR <- global chunk (l % CPR) ^ swizzle(row).  Wave w issues copies w, w + W, ...; the K swizzle of
+  // copy i's first row only flips chunk bits (V's is the same for every copy), so each lane's offset
+  // inside a stage's buffer is one register, i's rows a scalar offset.
   const int row_bytes = p.n_kv * HD * 2;
-  const int copy_row = wave * G::RPC + lane / G::CPR;
-  const uint32_t vk = uint32_t((lane / G::CPR) * row_bytes + (((lane % G::CPR) ^ G::swz_k(copy_row)) << 4));
-  const uint32_t vv = uint32_t((lane / G::CPR) * row_bytes + (((lane % G::CPR) ^ G::swz_v(copy_row)) << 4));
+  const int lr0 = lane / G::CPR;
+  const uint32_t vk = uint32_t(lr0 * row_bytes + (((lane % G::CPR) ^ G::swz_k(wave * G::RPC + lr0)) << 4));
+  const uint32_t vv = uint32_t(lr0 * row_bytes + (((lane % G::CPR) ^ G::swz_v(lr0)) << 4));
   // Element offset of a stage's rows of head h in the pools, for consecutive stages: one stage on from
   // the last, or the first of the next page.
   const int pmask = (1 << p.log2_page) - 1;
@@ -272,15 +377,16 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     off_k = int64_t(ok ? pid : 0) * p.page_stride + int64_t(T_k & pmask) * (p.n_kv * HD) + h * HD;
   };
   char* const ring_k = lds;
-  char* const ring_v = lds + pf::kRingK * G::STAGE;
-  // Iteration t issues the copies of K stage t + 5 and V stage t + 2 (t from -5), two of each per wave.
-  // Those of a stage that does not exist are issued too, with an empty buffer: they fetch nothing and
-  // write zeros to a free slot, and the loop has neither branches nor other counts to wait for.  A
-  // stage's page lookup serves its K copies and, three iterations later, its V copies: off1 .. off3
-  // hold the offsets of the stages in between, oldest first.
+  char* const ring_v = lds + kRing * G::STAGE;
+  // Iteration t issues the copies of K stage t + kLead + 2 and V stage t + kLead - 1 (from t = -kLead -
+  // 2), kCopies of each per wave.  Those of a stage that does not exist are issued too, with an empty
+  // buffer: they fetch nothing and write zeros to a free slot, and the loop has neither branches nor
+  // other counts to wait for.  A stage's page lookup serves its K copies and, three iterations later,
+  // its V copies: off1 .. off3 hold the offsets of the stages in between, oldest first.
   int64_t off1 = 0, off2 = 0, off3 = 0;
-  int slot_k = 0, slot_v = (pf::kRingV - 3) * G::STAGE;  // ring slots the next copies go to
-  int left_k = n, left_v = n + 3;                        // stages left to copy (V: from t = -5)
+  int slot_k = 0, slot_v = (kRing * 2 - 3) % kRing * G::STAGE;  // ring slots the next copies go to (V from stage -3)
+  int left_k = n, left_v = n + 3;                               // stages left to copy
+  auto next_slot = [](int slot) { return slot == (kRing - 1) * G::STAGE ? 0 : slot + G::STAGE; };
   auto next_stage = [&] {
     if (__builtin_expect((T_k & pmask) == 0 && left_k > 0, 0)) page_start();
     off1 = off2;
@@ -289,21 +395,22 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     off_k += stage_elems;
     T_k += TOK;
   };
-  auto copy_k = [&](int half) {
-    const int i = wave + 4 * half;
-    pf::copy_1k(p.k_cache + off3, left_k > 0 ? TOK * row_bytes : 0, vk, i * G::RPC * row_bytes, ring_k + slot_k + i * 1024);
-    if (half == 1) {
-      slot_k = slot_k == (pf::kRingK - 1) * G::STAGE ? 0 : slot_k + G::STAGE;
+  auto copy_k = [&](int k) {
+    const int i = wave + W * k;
+    pf::copy_1k(p.k_cache + off3, left_k > 0 ? TOK * row_bytes : 0, vk ^ uint32_t(G::swz_k(W * k * G::RPC) << 4),
+                i * G::RPC * row_bytes, ring_k + slot_k + i * 1024);
+    if (k == kCopies - 1) {
+      slot_k = next_slot(slot_k);
       --left_k;
     }
   };
   // off_v: off1 as it was before this iteration's next_stage()
-  auto copy_v = [&](int half, int64_t off_v) {
-    const int i = wave + 4 * half;
+  auto copy_v = [&](int k, int64_t off_v) {
+    const int i = wave + W * k;
     pf::copy_1k(p.v_cache + off_v, left_v > 0 && left_v <= n ? TOK * row_bytes : 0, vv, i * G::RPC * row_bytes,
                 ring_v + slot_v + i * 1024);
-    if (half == 1) {
-      slot_v = slot_v == (pf::kRingV - 1) * G::STAGE ? 0 : slot_v + G::STAGE;
+    if (k == kCopies - 1) {
+      slot_v = next_slot(slot_v);
       --left_v;
     }
   };
@@ -318,7 +425,7 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     kr[u][kk] = pf::lds_read16((k_lane ^ uint32_t(kk << 5)) + rd_k + u * 32 * G::ROWB);
   };
   auto next_k = [&] {
-    rd_k = rd_k + G::STAGE == lds_addr(ring_k) + pf::kRingK * G::STAGE ? lds_addr(ring_k) : rd_k + G::STAGE;
+    rd_k = rd_k + G::STAGE == lds_addr(ring_k) + kRing * G::STAGE ? lds_addr(ring_k) : rd_k + G::STAGE;
   };
   // Transpose reads (ds_read_b64_tr_b16): in each 16-lane group (g), lane 4 j + c names elements 32 dt
   // + 16 (g & 1) + 4 c .. + 3 of token row 16 s + 4 hi + j (then 8 rows further) and receives its
@@ -337,7 +444,7 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     vhi[at + DT] = lds_read_tr16_issue<S1 + H1>(a);
   };
   auto next_v = [&] {
-    rd_v = rd_v + G::STAGE == lds_addr(ring_v) + pf::kRingV * G::STAGE ? lds_addr(ring_v) : rd_v + G::STAGE;
+    rd_v = rd_v + G::STAGE == lds_addr(ring_v) + kRing * G::STAGE ? lds_addr(ring_v) : rd_v + G::STAGE;
   };
 
   // ---- state ----
@@ -389,9 +496,9 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
   // file.  The next scores go to sn (the last iteration's are of nothing and unused), stage t's
   // probabilities to pn.
   auto iterate = [&](int t, f32x16 (&s)[TT], f32x16 (&sn)[TT], const u32x4 (&pp)[2 * TT], u32x4 (&pn)[2 * TT]) {
-    // K of stage t + 2 and V of stage t - 1 landed (the last two iterations' copies may be in flight),
+    // K of stage t + 2 and V of stage t - 1 landed (the last kLead - 1 iterations' copies may be in flight),
     // this wave's own reads done
-    __builtin_amdgcn_s_waitcnt(0x0078);  // vmcnt(8) lgkmcnt(0)
+    pf::wait_vm<2 * kCopies * (kLead - 1), true>();
     raw_barrier();
     const int T0 = (t_first + t) * TOK;
     if (__builtin_expect(T0 + TOK - 1 > lim_min, 0)) {
@@ -423,7 +530,7 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
       product_qk(sn, i);
       if (i >= 2 && i < 6) read_v_issue(i - 2);
       exps(s, pn, i);
-      if (i == 1 || i == 6) copy_k(i / 6);
+      if (kCopies == 2 ? i == 1 || i == 6 : (i & 1) == 1) copy_k(kCopies == 2 ? i / 6 : i / 2);
       __builtin_amdgcn_sched_barrier(0);
     }
     next_v();
@@ -440,7 +547,7 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
       read_k(i);
       exps(s, pn, 8 + i);
       if (i > 0) max_step(sn, mx, i - 1);
-      if (i == 2 || i == 6) copy_v((i - 2) / 4, off_v);
+      if (kCopies == 2 ? i == 2 || i == 6 : (i & 1) == 1) copy_v(kCopies == 2 ? (i - 2) / 4 : i / 2, off_v);
       __builtin_amdgcn_sched_barrier(0);
     }
     max_step(sn, mx, 7);
@@ -458,22 +565,24 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
 
   if (n > 0) {
     // V of stage -1 reads as zero: iteration 0's PV products add nothing
-    rd_v = lds_addr(ring_v) + (pf::kRingV - 1) * G::STAGE;
+    rd_v = lds_addr(ring_v) + (kRing - 1) * G::STAGE;
     {
-      char* z = ring_v + (pf::kRingV - 1) * G::STAGE + threadIdx.x * 16;
+      char* z = ring_v + (kRing - 1) * G::STAGE + threadIdx.x * 16;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4*>(z + i * 4096) = u32x4{0u, 0u, 0u, 0u};
+      for (int i = 0; i < kCopies; ++i) *reinterpret_cast<u32x4*>(z + i * 1024 * W) = u32x4{0u, 0u, 0u, 0u};
     }
     page_start();
-    for (int t = -5; t < 0; ++t) {
+    auto copies = [&] {
       const int64_t off_v = off1;
       next_stage();
-      copy_k(0);
-      copy_k(1);
-      copy_v(0, off_v);
-      copy_v(1, off_v);
-    }
-    pf::wait_vm<14>();                   // K of stages 0 and 1 landed (20 copies, theirs 1, 2, 5 and 6)
+#pragma unroll
+      for (int k = 0; k < kCopies; ++k) copy_k(k);
+#pragma unroll
+      for (int k = 0; k < kCopies; ++k) copy_v(k, off_v);
+    };
+    for (int t = -kLead - 2; t < -1; ++t) copies();
+    // K of stages 0 and 1 landed, issued first in the first two of those iterations
+    pf::wait_vm<kCopies + 2 * kCopies * (kLead - 1)>();
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the zeroed slot
     raw_barrier();
     // The scores and probabilities alternate between two register sets, so the iterations go in pairs;
@@ -492,6 +601,9 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
 #pragma unroll
     for (int i = 0; i < 8; ++i) read_k(i);
     next_k();
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    raw_barrier();                       // K stage 0 is read: its slot takes iteration -1's copies
+    copies();
     int t = 0;
     if (n & 1) {
 #pragma unroll
@@ -561,10 +673,12 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
     return;
   }
   if constexpr (DEST == pf::kSplit) {
-    if (!whole) {
+    if (count > 1) {
       if (lo.real) {
-        const int64_t wrow = (int64_t((b * p.n_kv + h) * (int(gridDim.x) / p.max_splits) + xblk) * p.max_splits + split) *
-                                 pf::kRows + lo.r - blk_row0;
+        int64_t slot = int64_t(blockIdx.x);
+        if constexpr (W == pf::kWaves)
+          slot = int64_t((b * p.n_kv + h) * (int(gridDim.x) / p.max_splits) + xblk) * p.max_splits + split;
+        const int64_t wrow = slot * kRows + lo.r - blk_row0;
         float* dst = p.ws_o + wrow * HD + 4 * hi;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
@@ -590,21 +704,31 @@ __global__ __launch_bounds__(64 * pf::kWaves, 2) void prefill_tile_kernel(const 
   }
 }
 
-// Merge of a kSplit launch: grid (row block x HD / 8, KV head, sequence), 1024 / HD rows of an item per
+// Merge of a kSplit launch of ROWS-row blocks: grid (row block x ROWS HD / 1024, KV head, sequence), 1024 / HD rows of an item per
 // workgroup, one f32x4 of a row per thread.  Every range's load of a batch of 8 goes out before any is used.
-template <int HD>
+template <int HD, int ROWS>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p, int nx) {
   constexpr int TPR = HD / 4, RPW = 256 / TPR, B = 8;
-  constexpr int BLOCKS = pf::kRows / RPW;  // workgroups per item
+  constexpr int BLOCKS = ROWS / RPW;  // workgroups per item
   const int xblk = int(blockIdx.x) / BLOCKS, h = blockIdx.y, b = blockIdx.z;
   const int r = (int(blockIdx.x) % BLOCKS) * RPW + int(threadIdx.x) / TPR;  // row in the block
-  const int blk_row0 = xblk * pf::kRows;
-  int c, L;
-  seq_lengths(p, b, c, L);
-  const int count = pf::ranges_of(p, pf::stages_of<pf::Geo<HD>::TOK>(p, L, min(blk_row0 + pf::kRows, p.R) - 1)).count;
+  const int blk_row0 = xblk * ROWS;
   const int row = blk_row0 + r;
+  int count = 1;
+  int64_t w0;           // the first range's row in the workspace, and the rows to the next one's
+  int64_t w_step = ROWS;
+  if constexpr (ROWS == pf::kVerifyRows) {
+    const int first = p.ws_cnt[2 * b];
+    count = p.ws_cnt[2 * b + 1];
+    w0 = (int64_t(first) * p.n_kv + h) * ROWS + r;
+    w_step = int64_t(p.n_kv) * ROWS;
+  } else {
+    int c, L;
+    seq_lengths(p, b, c, L);
+    count = pf::ranges_of(p, pf::stages_of<pf::Geo<HD>::TOK>(p, L, min(blk_row0 + ROWS, p.R) - 1)).count;
+    w0 = int64_t((b * p.n_kv + h) * nx + xblk) * p.max_splits * ROWS + r;
+  }
   if (count <= 1 || row >= p.R) return;
-  const int64_t w0 = int64_t((b * p.n_kv + h) * nx + xblk) * p.max_splits * pf::kRows + r;
   const int d = (int(threadIdx.x) % TPR) * 4;
   float m = -INFINITY, l = 0.f;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -613,7 +737,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p, 
     f32x2 pm[B];
 #pragma unroll
     for (int k = 0; k < B; ++k) {
-      const int64_t w = w0 + int64_t(min(s0 + k, count - 1)) * pf::kRows;
+      const int64_t w = w0 + min(s0 + k, count - 1) * w_step;
       po[k] = *reinterpret_cast<const f32x4*>(p.ws_o + w * HD + d);
       pm[k] = *reinterpret_cast<const f32x2*>(p.ws_ml + 2 * w);
     }

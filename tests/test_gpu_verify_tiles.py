@@ -1,0 +1,72 @@
+"""Speculative verify on prefill_tile_kernel's two-wave form: 17 to 64 query rows per KV head, with the
+new rows appended by the ranges that cover them (a chunk that straddles two stages or two ranges, empty
+caches, new rows on a page boundary), ragged batches whose ranges differ in number, the largest batch of
+the rule and the one past it.  Caches bit-exact, outputs against the fp64 oracle, and against the
+balanced kernel the merge flag selects."""
+import numpy as np
+import pytest
+import torch
+
+import prism_amd
+from oracle import paged_attention as pa
+from pkv_testutil import make_paged_case
+
+pytestmark = pytest.mark.gpu
+
+# head_dim, n_heads, n_kv, page, s_q, contexts
+CASES = [
+    (128, 28, 4, 256, 5, [0, 27, 30, 253, 254, 4000]),
+    (128, 28, 4, 32, 3, [29, 30, 31, 500, 0]),
+    (128, 40, 8, 64, 4, [62, 1000, 7]),
+    (128, 8, 1, 256, 8, [1]),
+    (128, 7, 1, 256, 5, [9000, 3, 700]),
+    (64, 14, 2, 64, 5, [60, 61, 0, 3000, 700]),
+    (64, 16, 4, 256, 16, [255, 100, 2000]),
+    (128, 28, 4, 256, 5, [(i * 37) % 400 for i in range(64)]),
+    (128, 28, 4, 256, 5, [(i * 37) % 300 for i in range(65)]),  # past the rule: the balanced kernel
+]
+
+
+@pytest.mark.parametrize("append", [True, False])
+@pytest.mark.parametrize("case", CASES, ids=[f"hd{c[0]}-kv{c[2]}-p{c[3]}-s{c[4]}-b{len(c[5])}" for c in CASES])
+def test_verify_matches_oracle_and_balanced_kernel(gpu, case, append):
+    hd, nh, nk, page, s_q, ctx = case
+    cpu, d = make_paged_case(gpu, batch=len(ctx), ctx=ctx, page_size=page, n_kv=nk, n_heads=nh, head_dim=hd, s_q=s_q,
+                             seed=hd + nk + page + s_q)
+    for b, c in enumerate(ctx):   # stale slots behind the sequence hold NaN
+        end = c + s_q
+        for name in ("k_cache", "v_cache"):
+            for t in (cpu, d):
+                t[name][int(cpu["block_table"][b, (end - 1) // page]), (end - 1) % page + 1:] = float("nan")
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, shared_prefix_tokens=0)
+    k, v = (d["k"], d["v"]) if append else (None, None)
+    if not append:
+        d["cache_seqlens"] += s_q
+    other = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"].clone(), d["v_cache"].clone(), k, v, two_pass=True,
+                                              **kw)
+    out = torch.full((len(ctx), s_q, nh, hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+    prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], k, v, out=out, **kw)
+    torch.cuda.synchronize()
+    ref, kb, vb = pa.flash_attn_with_kvcache_ref(
+        cpu["q"], cpu["k_cache"], cpu["v_cache"], cpu["k"] if append else None, cpu["v"] if append else None,
+        cache_seqlens=d["cache_seqlens"].cpu(), block_table=cpu["block_table"], causal=True)
+    assert np.array_equal(pa.bf16_bits(d["k_cache"]), kb) and np.array_equal(pa.bf16_bits(d["v_cache"]), vb)
+    got = out.float().cpu().numpy()
+    assert np.isfinite(got).all()
+    err, near = np.abs(got - ref), np.abs(got - other.float().cpu().numpy())
+    few = np.array([[c + j + 1 <= 8 for j in range(s_q)] for c in ctx])
+    # a bf16 output is within half a unit of its value, P's own rounding within another: rows of a few
+    # keys reach one unit of the value where that passes 1e-2
+    assert err[~few].max(initial=0.0) <= 1e-2 and err.mean() <= 1e-3
+    assert (err[few] <= np.maximum(1e-2, np.abs(ref[few]) * 2.0 ** -7)).all()
+    assert (near <= np.maximum(1.6e-2, np.abs(ref) * 2.0 ** -6)).all()
+    assert prism_amd.read_status(gpu) == 0
+
+
+def test_verify_noalloc_is_bit_identical(gpu):
+    cpu, d = make_paged_case(gpu, batch=6, ctx=[0, 27, 30, 253, 254, 4000], page_size=256, n_kv=4, n_heads=28,
+                             head_dim=128, s_q=5, seed=5)
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, shared_prefix_tokens=0)
+    a = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], **kw)
+    b = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], noalloc=True, **kw)
+    assert torch.equal(a, b)
