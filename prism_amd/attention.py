@@ -240,6 +240,15 @@ def _workspace(device: torch.device, nbytes: int, stream: int, allow_static: boo
         return ws
 
 
+def _prefill_workspace(device: torch.device, stream: int, *sizes: int) -> torch.Tensor | None:
+    """The workspace of a prefill call that splits its keys, None where it does not.  A captured call
+    never does: its replays may run on any stream, beside eager calls that own the workspace."""
+    nbytes = _prefill_bytes(*sizes)
+    if nbytes == 0 or torch.cuda.is_current_stream_capturing():
+        return None
+    return _workspace(device, nbytes, stream)
+
+
 def _decode_flags(two_pass: bool | None, kernel: str, grid: int) -> int:
     flags = 0
     if two_pass is not None:
@@ -428,7 +437,7 @@ def flash_attn_with_kvcache(
     if (k is None) != (v is None):
         raise RuntimeError("k and v must both be given or both be None")
     if k is not None:
-        if k.shape[0] != batch or k.shape[1] != s_q or tuple(v.shape) != tuple(k.shape):
+        if k.shape[0] != batch or k.shape[1] != s_q or v.shape != k.shape:
             raise RuntimeError("k/v must be [B, s_q, n_kv, head_dim] matching q")
         ks = _rows(k, "k", n_kv, hd)
         vs = _rows(v, "v", n_kv, hd)
@@ -519,15 +528,26 @@ def flash_attn_with_kvcache(
             st.data_ptr(), stream)
         _lib.check(rc, "pkv_decode_attn")
     else:
-        # noalloc, or a capture without a sized workspace: the keys are not split
-        nbytes = 0 if noalloc else _prefill_bytes(batch, s_q, n_heads, n_kv, hd, page_size, max_blocks)
-        ws = _workspace(device, nbytes, stream, allow_static=True) if nbytes else None
+        # a table of fewer than 16 stages of 32 keys never splits: short prompts are host-bound (18 us a
+        # call), and asking the library costs them 0.3 us
+        ws = None if noalloc or max_blocks * page_size < 512 else \
+            _prefill_workspace(device, stream, batch, s_q, n_heads, n_kv, hd, page_size, max_blocks)
+        if ws is None:
+            rc = lib.pkv_prefill_attn(
+                q.data_ptr(), *qs, kp, *ks, vp, *vs,
+                k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
+                block_table.data_ptr(), block_table.stride(0), cache_seqlens.data_ptr(),
+                out.data_ptr(), *os_,
+                batch, s_q, n_heads, n_kv, hd, page_size, num_pages, max_blocks,
+                1 if causal else 0, scale, st.data_ptr(), stream)
+            _lib.check(rc, "pkv_prefill_attn")
+            return out
         rc = lib.pkv_prefill_attn_ws(
             q.data_ptr(), *qs, kp, *ks, vp, *vs,
             k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
             block_table.data_ptr(), block_table.stride(0), cache_seqlens.data_ptr(),
             out.data_ptr(), *os_,
-            ws.data_ptr() if ws is not None else 0, ws.numel() if ws is not None else 0,
+            ws.data_ptr(), ws.numel(),
             batch, s_q, n_heads, n_kv, hd, page_size, num_pages, max_blocks,
             1 if causal else 0, scale, st.data_ptr(), stream)
         _lib.check(rc, "pkv_prefill_attn_ws")
@@ -633,8 +653,7 @@ def prefill_attention(q, k_cache, v_cache, k=None, v=None, *, cache_seqlens, blo
     scale = float(softmax_scale) if softmax_scale is not None else 1.0 / math.sqrt(hd)
     lib = _lib.load()
     stream = _stream_ptr(q.device)
-    nbytes = _prefill_bytes(batch, s_q, n_heads, n_kv, hd, page_size, block_table.shape[1])
-    ws = _workspace(k_cache.device, nbytes, stream, allow_static=True)
+    ws = _prefill_workspace(k_cache.device, stream, batch, s_q, n_heads, n_kv, hd, page_size, block_table.shape[1])
     rc = lib.pkv_prefill_attn_ws(
         q.data_ptr(), *qs, kp, *ks, vp, *vs,
         k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),

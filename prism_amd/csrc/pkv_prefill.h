@@ -12,9 +12,9 @@
 // 16): a row's statistics live in two lanes, and registers 8 s .. 8 s + 7 packed to bf16 are the PV
 // operand of key step s as they stand, provided V^T names its tokens in the same order.
 //
-// Each tile's K and V rows are copied into LDS once per workgroup (8 buffer loads of 1 KiB each,
-// two of K and two of V per wave), K through a ring of 5 slots and V through one of 4, with counted
-// vmcnt waits and one raw barrier per tile.
+// Each stage's K and V rows are copied into LDS once per workgroup (8 buffer loads of 1 KiB each,
+// two of K and two of V per wave), through a ring of 4 slots of K and one of 4 of V (3 each in the
+// two-wave form), with counted vmcnt waits and one raw barrier per stage.
 //
 // What bounds it: the matrix pipe at 33 cycles per 32x32x16 product (16 products per tile and wave)
 // beside some 60 vector instructions of softmax and 24 LDS reads, and above that the card's power: a
@@ -704,8 +704,9 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
   }
 }
 
-// Merge of a kSplit launch of ROWS-row blocks: grid (row block x ROWS HD / 1024, KV head, sequence), 1024 / HD rows of an item per
-// workgroup, one f32x4 of a row per thread.  Every range's load of a batch of 8 goes out before any is used.
+// Merge of a kSplit launch of ROWS-row blocks: grid (row block x ROWS HD / 1024, KV head, sequence),
+// 1024 / HD rows of an item per workgroup, one f32x4 of a row per thread.  Every range's load of a batch
+// of 8 goes out before any is used.
 template <int HD, int ROWS>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const AttnParams p, int nx) {
   constexpr int TPR = HD / 4, RPW = 256 / TPR, B = 8;

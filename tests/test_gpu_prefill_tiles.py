@@ -1,6 +1,6 @@
 """prefill_tile_kernel at the sizes where its pipeline, its rows and its pages can go wrong: every
-count of key stages around the ring depths (an odd count starts with an empty stage, the V ring holds
-4 and the K ring 5), row blocks with a remainder, rows that see no key, pages of exactly one stage,
+count of key stages around the ring depths (an odd count does its first stage apart, the rings
+hold 4), row blocks with a remainder, rows that see no key, pages of exactly one stage,
 both head dims, with stale NaN behind every sequence.  Against the fp64 oracle at the bf16 tolerance."""
 import numpy as np
 import pytest
@@ -125,19 +125,25 @@ def test_prefill_split_keys_matches_unsplit_and_oracle(gpu, case, append):
     assert prism_amd.read_status(gpu) == 0
 
 
-def test_prefill_captured_without_a_workspace_runs_unsplit(gpu):
-    """A capture sizes no workspace of its own: the captured call and its replays give the eager
-    unsplit result."""
+def test_prefill_captured_runs_unsplit(gpu):
+    """A captured call takes no workspace, also where eager calls have sized one (its replays may run
+    beside them on other streams): its replays give the unsplit result."""
     cpu, d = make_paged_case(gpu, batch=1, ctx=[900], page_size=256, n_kv=4, n_heads=28, head_dim=128, s_q=40, seed=1)
-    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, noalloc=True)
-    want = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], **kw)
-    out = torch.empty_like(want)
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True)
+    args = d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"]
+    want = prism_amd.flash_attn_with_kvcache(*args, noalloc=True, **kw)
+    split = prism_amd.flash_attn_with_kvcache(*args, **kw)
+    assert not torch.equal(split, want)  # other fp32 sum orders: the eager call does split
+    out, out2 = torch.empty_like(want), torch.empty_like(want)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], out=out, **kw)
+        prism_amd.flash_attn_with_kvcache(*args, out=out, **kw)
+        prism_amd.prefill_attention(*args, out=out2, **kw)
     for _ in range(3):
         out.zero_()
+        out2.zero_()
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out, want)
+        assert torch.equal(out, want) and torch.equal(out2, want)
+        assert torch.equal(prism_amd.flash_attn_with_kvcache(*args, **kw), split)
