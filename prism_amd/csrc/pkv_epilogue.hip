@@ -143,8 +143,8 @@ __global__ __launch_bounds__(256) void rope_qk_kernel(const RopeParams p) {
     float o1[8], o2[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      o1[e] = bf16r(bf16r(x1[e] * c1[e]) + bf16r(-x2[e] * s1[e]));
-      o2[e] = bf16r(bf16r(x2[e] * c2[e]) + bf16r(x1[e] * s2[e]));
+      o1[e] = bf16r(x1[e] * c1[e]) + bf16r(-x2[e] * s1[e]);
+      o2[e] = bf16r(x2[e] * c2[e]) + bf16r(x1[e] * s2[e]);
     }
     const u32x4 v1 = pack8(o1), v2 = pack8(o2);
     if (!is_k) {
@@ -245,7 +245,15 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const NormParams p) {
 
 // ---------------------------------------------------------------------------------------------
 // SiLU(gate) * up over rows of m values: out = bf16(bf16(silu(g)) * u), the two roundings of the
-// reference's F.silu(gu[..., :m]) * gu[..., m:] on bf16 tensors.  Grid-stride over 16-byte chunks.
+// reference's F.silu(gu[..., :m]) * gu[..., m:] on bf16 tensors.  Grid (256 16-byte chunks of a row,
+// rows).  Memory bounds it: 4096 x 13824 is 340 MB in 58 us (5.9 TB/s).  A 64-bit division per chunk to
+// find the row and eight IEEE divisions held it at 60.
+//
+// STREAM reads gate and up non-temporally, for launches that read more than the eight 4 MiB L2s hold
+// (kStreamBytes).  14B, plain / non-temporal: right behind the launch that wrote them, 2048 rows 25.2 /
+// 24.0 us, 4096 45.7 / 43.6, 8192 148 / 102; from memory, 4096 58.0 / 54.0.  Below the line an input
+// that is still in the L2s would be lost there: 512 rows 5.5 / 7.0; at 768 (40 MiB) both take 10.5.
+// rope_qk_kernel keeps plain loads: behind its producer 4096 rows take 17.5 / 18.3.
 // ---------------------------------------------------------------------------------------------
 struct SiluParams {
   const uint16_t* gate;
@@ -258,22 +266,43 @@ struct SiluParams {
   int m;
 };
 
+constexpr int64_t kStreamBytes = int64_t(32) << 20;
+
+// g / d for |g| < 80 (d = 1 + exp(-g) then stays below 6e34, and no step overflows or is subnormal): the
+// reciprocal to 1 ulp, and the quotient corrected by its remainder (which turns -0 into 0: the sign is
+// put back).  5 instructions where the IEEE division takes 10, and its very quotient for every bf16 g,
+// with the reciprocal a ulp off either way.
+__device__ __forceinline__ float div_bounded(float g, float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float q = g * r;
+  return copysignf(fmaf(fmaf(-d, q, g), r, q), g);
+}
+
+template <bool STREAM>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const SiluParams p) {
-  const int cpr = p.m / 8;
-  const int64_t total = p.rows * cpr;
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += stride) {
-    const int64_t r = i / cpr;
-    const int c = int(i - r * cpr);
-    float gf[8], uf[8], o[8];
-    unpack8(ld16(p.gate + r * p.g_stride + 8 * c), gf);
-    unpack8(ld16(p.up + r * p.u_stride + 8 * c), uf);
+  const int c = int(blockIdx.x) * 256 + int(threadIdx.x);
+  if (c >= p.m / 8) return;
+  auto load = [](const uint16_t* src) {
+    return STREAM ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src)) : ld16(src);
+  };
+  for (int64_t r = blockIdx.y; r < p.rows; r += gridDim.y) {
+    float gf[8], uf[8], s[8];
+    unpack8(load(p.gate + r * p.g_stride + 8 * c), gf);
+    unpack8(load(p.up + r * p.u_stride + 8 * c), uf);
+    float big = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float s = bf16r(gf[e] / (1.f + __expf(-gf[e])));
-      o[e] = s * uf[e];
+    for (int e = 0; e < 8; ++e) big = fmaxf(big, fabsf(gf[e]));
+    if (__builtin_expect(big < 80.f, 1)) {  // a NaN passes, and stays one
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] = div_bounded(gf[e], 1.f + __expf(-gf[e]));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] = gf[e] / (1.f + __expf(-gf[e]));
     }
-    __builtin_nontemporal_store(pack8(o), reinterpret_cast<u32x4*>(p.out + r * p.o_stride + 8 * c));
+    unpack8(pack8(s), s);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] *= uf[e];
+    __builtin_nontemporal_store(pack8(s), reinterpret_cast<u32x4*>(p.out + r * p.o_stride + 8 * c));
   }
 }
 
@@ -402,8 +431,8 @@ extern "C" int pkv_silu_mul(const void* gate, int64_t g_stride, const void* up, 
   p.o_stride = o_stride;
   p.rows = rows;
   p.m = m;
-  const int64_t want = (total + 255) / 256;
-  const int blocks = int(want < 16384 ? want : 16384);
-  silu_mul_kernel<<<blocks, 256, 0, static_cast<hipStream_t>(stream)>>>(p);
+  const dim3 grid(unsigned((m / 8 + 255) / 256), unsigned(rows < 65535 ? rows : 65535));
+  auto* kernel = total * 32 > kStreamBytes ? silu_mul_kernel<true> : silu_mul_kernel<false>;
+  kernel<<<grid, 256, 0, static_cast<hipStream_t>(stream)>>>(p);
   return check_launch(fn);
 }

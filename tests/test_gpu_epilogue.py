@@ -203,3 +203,35 @@ def test_silu_mul_matches_reference(gpu):
     _ulp_close(out, ref, "silu_mul", 1.0)
     exact = np.mean(out.float().cpu().numpy() == ref)
     assert exact > 0.99, f"only {exact:.4f} of outputs bit-exact"
+
+
+@pytest.mark.parametrize("rows,m", [(1, 8), (3, 2040), (2, 2056), (65537, 8), (1025, 8192)])
+def test_silu_mul_edges(gpu, rows, m):
+    """One chunk, a workgroup's 256 chunks less and plus one, more rows than the grid holds, just past the
+    size that reads non-temporally; gates on both
+    sides of the division's bound (|g| = 80), where exp overflows (-89) and past bf16's range of silu."""
+    gu = _rand((rows, 2 * m), rows + m, 3.0)
+    edge = torch.tensor([79.5, 80.0, -79.5, -80.0, -87.0, -89.0, 3e38, 0.0], dtype=torch.bfloat16)
+    gu[rows - 1, m - 8:m] = edge
+    gu[rows - 1, 2 * m - 8:] = 0.5
+    ref = ep.silu_mul_ref(gu[:, :m].float().numpy(), gu[:, m:].float().numpy())
+    d = gu.to(gpu)
+    out = prism_amd.silu_mul(d[:, :m], d[:, m:])
+    torch.cuda.synchronize()
+    got = out.float().cpu().numpy()
+    # below 2^-100 (gates under -70) the reference and the kernel's exp agree to fp32's range, not its ulp
+    tiny = np.abs(ref) < 2.0 ** -100
+    assert (np.abs(got - ref)[tiny] <= 2.0 ** -100).all()
+    _ulp_close(torch.from_numpy(np.where(tiny, 0, got)), np.where(tiny, 0, ref), f"silu_mul {rows}x{m}", 1.0)
+
+
+def test_silu_mul_infinities_and_nan(gpu):
+    g = torch.tensor([float("inf"), -float("inf"), float("nan"), 1.0, float("nan"), 100.0, -100.0, 2.0],
+                     dtype=torch.bfloat16)
+    out = prism_amd.silu_mul(g.to(gpu)[None], torch.ones(1, 8, dtype=torch.bfloat16, device=gpu))[0].float().cpu()
+    # -inf / inf: NaN, as the plain division (and torch's silu in float) gives
+    assert out[0] == float("inf") and out[[1, 2, 4]].isnan().all()
+    assert out[5] == 100.0 and abs(float(out[6])) < 1e-30 and abs(float(out[3]) - 0.7311) < 4e-3
+    zero = torch.tensor([[0.0, -0.0] * 4], dtype=torch.bfloat16, device=gpu)
+    out = prism_amd.silu_mul(zero, torch.ones_like(zero))
+    assert torch.equal(out.signbit(), zero.signbit()) and (out == 0).all()
