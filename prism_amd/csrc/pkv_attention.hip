@@ -3078,12 +3078,15 @@ static size_t ws_bytes_prefill(int batch, int64_t R, int n_kv, int head_dim, int
 // serial chain per wave at one wave per SIMD, with a 1.8-2.4 us segment start per sequence and a
 // 7-8 us merge launch; this form runs six waves per CU and starts a range in about 2.5 us.  Per call,
 // lean / tiles: 7B B = 8 26.4 / 20.1 us, B = 32 42.5 / 39.7, B = 64 over a shared 2048-token prefix
-// 57.8 / 50.2, 14B B = 16 42.4 / 41.8, one TP-4 shard B = 16 32.2 / 19.7, 0.5B B = 64 40.0 / 27.1; ahead
-// or level at each of 34 random draws up to one (sequence, KV head) per CU.  Past that the ranges no
-// longer fit one round: 7B B = 128 58.4 / 64.1, so the rule ends there.
-// It takes the calls decode_lean_kernel would take
-// with more than 16 query rows per KV head (both round P to bf16 once), unless a flag asks for a merge
-// or a grid.  Key ranges per KV head: about one round of kVerifyPerCu workgroups per CU over all heads.
+// 57.8 / 50.2, 14B B = 16 42.4 / 41.8; ahead or level at each random draw up to one (sequence, KV head)
+// per CU.  Past that the ranges no longer fit one round: 7B B = 128 58.4 / 64.1, so the rule ends there.
+// It takes the calls of decode_lean_kernel's geometry of four KV heads at head_dim 128, where both round
+// P to bf16 once (error against 64 bits 2.2-2.4e-3 on either), with more than 16 query rows per KV head,
+// unless a flag asks for a merge or a grid.  The others are more exact on decode_lean_kernel and stay
+// there, though slower: head_dim 64 keeps P as a bf16 pair (0.5B B = 6 1.7e-3 / 2.3e-3; B = 64 40.0 /
+// 27.1 us), and one or two KV heads run 4 or 2 phases with a row maximum each (a TP-4 shard at B = 3
+// 2.1e-3 / 2.3e-3; B = 16 32.2 / 19.7 us).  Key ranges per KV head: about one round of kVerifyPerCu
+// workgroups per CU over all heads.
 constexpr size_t kScratchBytes = size_t(48) << 20;  // pkv_decode_attn_noalloc's static scratch
 static int verify_target(int n_kv) {
   const int t = pf::kVerifyPerCu * device_cu_count() / n_kv;
@@ -3098,16 +3101,15 @@ static size_t ws_bytes_verify(int batch, int n_kv, int head_dim) {
 // Only where the ranges fit the static scratch, so that a call takes the same kernel with and without
 // a workspace of its own.
 static bool use_verify_tiles(int batch, int n_kv, int head_dim, int R, int page_size, bool lean, int32_t flags) {
-  return lean && R > 16 && page_size >= (head_dim == 128 ? pf::Geo<128>::TOK : pf::Geo<64>::TOK) &&
+  return lean && lean_geom(head_dim, n_kv) == kGeom128x4 && R > 16 && page_size >= pf::Geo<128>::TOK &&
          (flags & ~PKV_DECODE_RESET_COUNTERS) == 0 && int64_t(batch) * n_kv <= device_cu_count() &&
          ws_bytes_verify(batch, n_kv, head_dim) <= kScratchBytes;
 }
-template <int HD>
 static void launch_verify_tiles(const AttnParams& p, int batch, hipStream_t stream) {
-  prefill_tile_kernel<HD, pf::kSplit, pf::kVerifyWaves>
+  prefill_tile_kernel<128, pf::kSplit, pf::kVerifyWaves>
       <<<unsigned(verify_slots(batch, p.n_kv)), 64 * pf::kVerifyWaves, 0, stream>>>(p);
-  prefill_merge_kernel<HD, pf::kVerifyRows>
-      <<<dim3((p.R * HD + 1023) / 1024, p.n_kv, batch), 256, 0, stream>>>(p, 1);
+  prefill_merge_kernel<128, pf::kVerifyRows>
+      <<<dim3((p.R * 128 + 1023) / 1024, p.n_kv, batch), 256, 0, stream>>>(p, 1);
 }
 
 // splits > 1 needs ws_o / ws_ml.
@@ -3302,10 +3304,7 @@ static int decode_attn(const char* fn, bool use_scratch, const void* q, int64_t 
     p.ws_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
     p.ws_ml = p.ws_o + size_t(verify_slots(batch, n_kv)) * pf::kVerifyRows * head_dim;
     p.ws_cnt = reinterpret_cast<int32_t*>(p.ws_ml + size_t(verify_slots(batch, n_kv)) * pf::kVerifyRows * 2);
-    if (head_dim == 128)
-      launch_verify_tiles<128>(p, batch, s);
-    else
-      launch_verify_tiles<64>(p, batch, s);
+    launch_verify_tiles(p, batch, s);
     return check_launch(fn);
   }
   if (lean) {

@@ -136,8 +136,8 @@ __device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
 
 // Verify's ranges.  The stages of all sequences, sequence after sequence, are cut into ranges of one
-// length (`chunk`: about lean_grid ranges for each KV head, at least kMinVerifyStages stages each: 2 cost
-// the TP-4 shard 12 us, 4 to 6 are level), each inside
+// length (`chunk`: about lean_grid ranges for each KV head, at least kMinVerifyStages stages each: 4 to 6
+// are level), each inside
 // one sequence: a ragged batch keeps every workgroup at the same work, whatever the longest sequence.
 // Range w of KV head h is workgroup w n_kv + h, so that each XCD's L2 serves few heads (a cached prefix
 // that the batch shares is then read once per XCD and head).

@@ -1,7 +1,8 @@
 """Speculative verify on prefill_tile_kernel's two-wave form: 17 to 64 query rows per KV head, with the
 new rows appended by the ranges that cover them (a chunk that straddles two stages or two ranges, empty
 caches, new rows on a page boundary), ragged batches whose ranges differ in number, the largest batch of
-the rule and the one past it.  Caches bit-exact, outputs against the fp64 oracle, and against the
+the rule and the one past it, and the head counts and dims that the balanced kernel keeps because it is
+more exact there.  Caches bit-exact, outputs against the fp64 oracle, and against the
 balanced kernel the merge flag selects."""
 import numpy as np
 import pytest
@@ -18,8 +19,9 @@ CASES = [
     (128, 28, 4, 256, 5, [0, 27, 30, 253, 254, 4000]),
     (128, 28, 4, 32, 3, [29, 30, 31, 500, 0]),
     (128, 40, 8, 64, 4, [62, 1000, 7]),
-    (128, 8, 1, 256, 8, [1]),
-    (128, 7, 1, 256, 5, [9000, 3, 700]),
+    (128, 32, 4, 256, 8, [1]),
+    (128, 28, 4, 256, 5, [9000, 3, 700]),
+    (128, 7, 1, 256, 5, [9000, 3, 700]),  # the balanced kernel, and the next two
     (64, 14, 2, 64, 5, [60, 61, 0, 3000, 700]),
     (64, 16, 4, 256, 16, [255, 100, 2000]),
     (128, 28, 4, 256, 5, [(i * 37) % 400 for i in range(64)]),
@@ -61,6 +63,18 @@ def test_verify_matches_oracle_and_balanced_kernel(gpu, case, append):
     assert (err[few] <= np.maximum(1e-2, np.abs(ref[few]) * 2.0 ** -7)).all()
     assert (near <= np.maximum(1.6e-2, np.abs(ref) * 2.0 ** -6)).all()
     assert prism_amd.read_status(gpu) == 0
+
+
+@pytest.mark.parametrize("hd,nh,nk", [(64, 14, 2), (64, 16, 4), (128, 7, 1), (128, 14, 2)])
+def test_verify_keeps_the_more_exact_kernel(gpu, hd, nh, nk):
+    """Where the balanced kernel holds P as a bf16 pair (head_dim 64) or a maximum per phase (one or two
+    KV heads), the call is its launch: bit-identical to the one a merge flag selects."""
+    cpu, d = make_paged_case(gpu, batch=6, ctx=[0, 27, 30, 253, 254, 600], page_size=256, n_kv=nk, n_heads=nh,
+                             head_dim=hd, s_q=5, seed=5)
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, shared_prefix_tokens=0)
+    a = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], **kw)
+    b = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], two_pass=True, **kw)
+    assert torch.equal(a, b)
 
 
 def test_verify_noalloc_is_bit_identical(gpu):
