@@ -19,7 +19,8 @@ Calls are asynchronous on the caller's current stream, allocate only ``out`` (an
 grow-only split-K workspace per device and stream), and can be captured in a HIP graph once an
 eager call on the device has sized the workspace (on any stream: a capture stream without one of
 its own shares the largest, as Prism's warm-up on its current stream then capture on a new stream
-needs).
+needs).  Eager prefill calls that split their keys keep their partials in a second workspace per
+device and stream, which captured calls never use.
 """
 from __future__ import annotations
 
@@ -34,6 +35,9 @@ from . import _lib
 _BF16 = torch.bfloat16
 _ws_lock = threading.Lock()
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
+# Prefill's key-range partials have buffers of their own: a capture borrows decode's largest one
+# (_workspace), and its replays must not share it with eager prefills on another stream.
+_prefill_workspaces: dict[tuple[int, int], torch.Tensor] = {}
 _captured: set[int] = set()         # data_ptr of every workspace handed to a call under graph capture
 _retired: list[torch.Tensor] = []   # outgrown workspaces a captured graph may still use
 _status: dict[int, torch.Tensor] = {}
@@ -241,12 +245,18 @@ def _workspace(device: torch.device, nbytes: int, stream: int, allow_static: boo
 
 
 def _prefill_workspace(device: torch.device, stream: int, *sizes: int) -> torch.Tensor | None:
-    """The workspace of a prefill call that splits its keys, None where it does not.  A captured call
-    never does: its replays may run on any stream, beside eager calls that own the workspace."""
+    """The workspace of a prefill call that splits its keys, None where it does not: one per (device,
+    stream), grow-only, and never handed to a capture.  A captured prefill does not split, because its
+    replays may run on any stream, beside eager calls that own the workspace."""
     nbytes = _prefill_bytes(*sizes)
     if nbytes == 0 or torch.cuda.is_current_stream_capturing():
         return None
-    return _workspace(device, nbytes, stream)
+    key = (_dev_index(device), stream)
+    with _ws_lock:
+        ws = _prefill_workspaces.get(key)
+        if ws is None or ws.numel() < nbytes:
+            ws = _prefill_workspaces[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return ws
 
 
 def _decode_flags(two_pass: bool | None, kernel: str, grid: int) -> int:

@@ -12,6 +12,7 @@ import torch
 from hypothesis import given, settings
 from hypothesis import strategies as st
 
+import prism_amd.attention as attn
 import prism_amd.kv_cache as kvm
 from oracle import page_ops
 from oracle.paged_attention import bf16_bits
@@ -306,3 +307,25 @@ def test_status_error_names_every_bit():
     assert e.bits == bits and e.device == 3 and isinstance(e, RuntimeError)
     assert "BAD_PAGE" in str(e) and "MERGE_TIMEOUT" in str(e) and "cuda:3" in str(e)
     assert "PARTIAL_RANGE" not in str(e)
+
+
+def test_a_capture_never_borrows_a_prefill_workspace(monkeypatch):
+    """Eager prefill sizes a large buffer on stream B, a decode warm-up a smaller one on stream A; a capture
+    on stream C takes A's, and prefills on A (before or after the capture) leave it alone."""
+    monkeypatch.setattr(attn, "_workspaces", {})
+    monkeypatch.setattr(attn, "_prefill_workspaces", {}, raising=False)
+    monkeypatch.setattr(attn, "_captured", set())
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    dev, A, B, C = torch.device("cpu", 0), 11, 22, 33
+    sizes = (1, 150, 28, 4, 128, 256, 15)  # 150 tokens onto 3500 at the 7B shape
+    pre = attn._prefill_workspace(dev, B, *sizes)
+    pre_a = attn._prefill_workspace(dev, A, *sizes)
+    dec = attn._workspace(dev, 2 << 20, A)
+    assert pre.numel() > dec.numel() and pre.data_ptr() != pre_a.data_ptr()
+    capturing[0] = True
+    got = attn._workspace(dev, 2 << 20, C)
+    assert got.data_ptr() == dec.data_ptr()
+    assert attn._prefill_workspace(dev, C, *sizes) is None and attn._prefill_workspace(dev, A, *sizes) is None
+    capturing[0] = False
+    assert attn._prefill_workspace(dev, A, *sizes).data_ptr() == pre_a.data_ptr() != got.data_ptr()
