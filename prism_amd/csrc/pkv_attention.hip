@@ -3525,10 +3525,13 @@ extern "C" int pkv_cascade_attn(const void* q, int64_t q_sb, int64_t q_ss, int64
 extern "C" size_t pkv_prefill_workspace_bytes(int32_t batch, int32_t s_q, int32_t n_heads, int32_t n_kv,
                                               int32_t head_dim, int32_t page_size, int32_t max_blocks) {
   using namespace pkv;
-  if (batch <= 0 || s_q <= 0 || n_kv <= 0 || n_heads <= 0 || max_blocks <= 0 || page_size <= 0 ||
-      (head_dim != 64 && head_dim != 128))
+  // the sizes pkv_prefill_attn rejects need no workspace (n_heads < n_kv would be no row blocks at all)
+  if (batch <= 0 || batch > 65535 || s_q <= 0 || n_kv <= 0 || n_kv > 65535 || n_heads <= 0 || n_heads % n_kv ||
+      max_blocks <= 0 || !is_pow2(page_size) || page_size < 16 ||
+      int64_t(max_blocks) * page_size > (int64_t(1) << 27) || (head_dim != 64 && head_dim != 128))
     return 0;
   const int64_t R = int64_t(s_q) * (n_heads / n_kv);
+  if (R > (int64_t(1) << 30)) return 0;
   return ws_bytes_prefill(batch, R, n_kv, head_dim, prefill_splits(batch, R, n_kv, head_dim, page_size, max_blocks));
 }
 

@@ -112,6 +112,17 @@ def test_workspace_bytes_arithmetic(lib):
         assert f(2, 1, nh, nkv, hd, 256, 8, 0) == max(65536 + 2 * 256 * 4 * R * 260, per_head)
 
 
+@pytest.mark.parametrize("sizes", [
+    (1, 40, 2, 4, 128, 256, 8),                 # fewer query heads than KV heads: no row blocks to divide by
+    (1, 40, 30, 4, 128, 256, 8),
+    (1, 1 << 30, 28, 4, 128, 256, 8),           # more query rows than a call takes
+    (1 << 30, 1 << 30, 1 << 30, 1 << 30, 128, 256, 8),
+    (1, 40, 28, 4, 96, 256, 8), (1, 40, 28, 4, 128, 48, 8), (1, 40, 28, 4, 128, 256, (1 << 19) + 1),
+])
+def test_prefill_workspace_bytes_of_rejected_sizes_is_zero(lib, sizes):
+    assert lib.pkv_prefill_workspace_bytes(*sizes) == 0
+
+
 def test_copy_and_gather_argument_errors(lib):
     rc = lib.pkv_copy_pages(A16, A16, 2, A16, A16, None, 3, 1000, 1 << 18, 1024, 256, 10, 10, None, None)
     assert rc == _lib.PKV_EINVAL and "pkv_copy_pages" in lib.pkv_last_error().decode()

@@ -245,3 +245,11 @@ def test_no_append_causal_verify_cuts_the_automatic_cascade_prefix(gpu, prefix, 
     ref, _, _ = pa.flash_attn_with_kvcache_ref(q.cpu(), kc, vc, cache_seqlens=sl.cpu(),
                                                block_table=bt.cpu().clamp(min=0), causal=True)
     assert_attn_close(out, ref, f"no-append causal verify, prefix {prefix}, s_q {s_q}")
+
+
+def test_prefill_head_mismatch_raises(gpu):
+    # fewer query heads than KV heads, with pages for many keys: an error, as from the kernel's own checks
+    _, d = make_paged_case(gpu, batch=1, ctx=[2000], page_size=256, n_kv=4, n_heads=2, head_dim=128, s_q=40, seed=1)
+    with pytest.raises(RuntimeError, match="n_heads"):
+        prism_amd.prefill_attention(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"],
+                                    cache_seqlens=d["cache_seqlens"], block_table=d["block_table"])
