@@ -255,7 +255,11 @@ def _prefill_workspace(device: torch.device, stream: int, *sizes: int) -> torch.
     with _ws_lock:
         ws = _prefill_workspaces.get(key)
         if ws is None or ws.numel() < nbytes:
-            ws = _prefill_workspaces[key] = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            try:
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            except torch.OutOfMemoryError:
+                return None   # pools that fill the card: the call runs unsplit, which needs no workspace
+            _prefill_workspaces[key] = ws
         return ws
 
 

@@ -329,3 +329,17 @@ def test_a_capture_never_borrows_a_prefill_workspace(monkeypatch):
     assert attn._prefill_workspace(dev, C, *sizes) is None and attn._prefill_workspace(dev, A, *sizes) is None
     capturing[0] = False
     assert attn._prefill_workspace(dev, A, *sizes).data_ptr() == pre_a.data_ptr() != got.data_ptr()
+
+
+def test_a_prefill_without_memory_for_its_workspace_runs_unsplit(monkeypatch):
+    monkeypatch.setattr(attn, "_prefill_workspaces", {})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    dev, sizes = torch.device("cpu", 0), (1, 150, 28, 4, 128, 256, 15)
+
+    def full(*a, **k):
+        raise torch.OutOfMemoryError("no memory")
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", full)
+        assert attn._prefill_workspace(dev, 1, *sizes) is None
+    assert attn._prefill_workspace(dev, 1, *sizes) is not None
