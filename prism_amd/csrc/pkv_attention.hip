@@ -3077,16 +3077,19 @@ static size_t ws_bytes_prefill(int batch, int64_t R, int n_kv, int head_dim, int
 // Speculative verify on prefill_tile_kernel's two-wave form.  decode_lean_kernel's verify rows are one
 // serial chain per wave at one wave per SIMD, with a 1.8-2.4 us segment start per sequence and a
 // 7-8 us merge launch; this form runs six waves per CU and starts a range in about 2.5 us.  Per call,
-// lean / tiles: 7B B = 8 26.4 / 20.1 us, B = 32 42.5 / 39.7, B = 64 over a shared 2048-token prefix
-// 57.8 / 50.2, 14B B = 16 42.4 / 41.8; ahead or level at each random draw up to one (sequence, KV head)
-// per CU.  Past that the ranges no longer fit one round: 7B B = 128 58.4 / 64.1, so the rule ends there.
-// It takes the calls of decode_lean_kernel's geometry of four KV heads at head_dim 128, where both round
-// P to bf16 once (error against 64 bits 2.2-2.4e-3 on either), with more than 16 query rows per KV head,
-// unless a flag asks for a merge or a grid.  The others are more exact on decode_lean_kernel and stay
-// there, though slower: head_dim 64 keeps P as a bf16 pair (0.5B B = 6 1.7e-3 / 2.3e-3; B = 64 40.0 /
-// 27.1 us), and one or two KV heads run 4 or 2 phases with a row maximum each (a TP-4 shard at B = 3
-// 2.1e-3 / 2.3e-3; B = 16 32.2 / 19.7 us).  Key ranges per KV head: about one round of kVerifyPerCu
-// workgroups per CU over all heads.
+// five query rows, lean / tiles: 7B B = 8 25.3 / 20.1 us, B = 32 36.8 / 33.0, B = 64 72.9 / 69.7, B = 64
+// over a shared 2048-token prefix 55.8 / 50.0, 14B B = 16 36.7 / 36.6, B = 32 61.7 / 59.2.  Past one
+// (sequence, KV head) per CU the ranges no longer fit one round: 7B B = 128 124.6 / 133.2, shared 95.2 /
+// 96.2, so the rule ends there.
+// Its ranges are longer than decode_lean_kernel's shares, so fewer keys meet a running maximum of their
+// own, where P is exactly 1: rounded to bf16 once, P would be further off (7B, 2 to 12 short contexts:
+// 2.04e-3 from 64 bits on decode_lean_kernel, 2.24e-3 here).  It is a bf16 hi + lo pair instead, 1.66e-3
+// on every call, which is the output's own rounding; the second product of a stage costs 0 to 2%.
+// It takes the calls of decode_lean_kernel's geometry of four KV heads at head_dim 128 with more than 16
+// query rows per KV head, unless a flag asks for a merge or a grid.  head_dim 64 and one or two KV heads
+// stay on decode_lean_kernel: there this form has been timed with P rounded once only (0.5B B = 64 40.0 /
+// 27.1 us, a TP-4 shard at B = 16 32.2 / 19.7), which is less exact than what they have.  Key ranges per
+// KV head: about one round of kVerifyPerCu workgroups per CU over all heads.
 constexpr size_t kScratchBytes = size_t(48) << 20;  // pkv_decode_attn_noalloc's static scratch
 static int verify_target(int n_kv) {
   const int t = pf::kVerifyPerCu * device_cu_count() / n_kv;

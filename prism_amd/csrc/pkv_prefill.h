@@ -120,6 +120,15 @@ __device__ __forceinline__ float add_pair(uint32_t pair, float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), ones, acc, false);
 }
 
+// Two probabilities as bf16 pairs hi + lo: hi truncated, so that lo is not negative, and lo a 2^-23 of p
+// too large, so that it is not zero either where p is not: an infinite V stays that infinity under both.
+__device__ __forceinline__ uint32_t split_pair(float a, float b, uint32_t& hi) {
+  const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+  constexpr float kUp = 1.f + 0x1p-23f;
+  hi = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+  return pack_bf16x2(fmaf(a, kUp, -__uint_as_float(ua & 0xFFFF0000u)), fmaf(b, kUp, -__uint_as_float(ub & 0xFFFF0000u)));
+}
+
 // Over the two lanes {l, l ^ 32} that hold a row.
 __device__ __forceinline__ float sum_halves(float v) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -198,7 +207,9 @@ __device__ __forceinline__ void verify_ranges(const AttnParams& p, const VerifyP
 // log-sum-exp) in workspace slot 2 G + b S + z of each row.
 //
 // W waves own 32 W rows.  W = 2 (kSplit only) is speculative verify: one row block per (sequence, KV
-// head); each range appends the new rows it covers itself, before it copies them.
+// head); each range appends the new rows it covers itself, before it copies them; P is a bf16 pair (two
+// PV products: the launch is bound by range starts and copies, 64 branches of one 2048-token prompt 49
+// -> 50 us a call).
 template <int HD, int DEST, int W = pf::kWaves>
 __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParams p) {
   using G = pf::Geo<HD>;
@@ -208,6 +219,8 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
   constexpr int kCopies = 8 / W;                  // copies of a K (or V) stage per wave
   constexpr int TT = G::TT, DT = G::DT, KK = G::KK, TOK = G::TOK;
   constexpr bool CASCADE = DEST == pf::kCascade;
+  constexpr bool PAIR = W != pf::kWaves;          // P as bf16 hi + lo
+  constexpr int NP = PAIR ? 4 * TT : 2 * TT;      // PV operands of a stage: hi (then lo) of each key step
   __shared__ __attribute__((aligned(16))) char lds[2 * kRing * G::STAGE];
 
   const int lane = threadIdx.x & 63;
@@ -462,16 +475,18 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
       for (int r = 0; r < 16; ++r) s[u][r] = 0.f;
     s[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kr[u][kk]), qf[kk], s[u], 0, 0, 0);
   };
-  auto product_pv = [&](const u32x4 (&pk)[2 * TT], int i) {
+  auto product_pv = [&](const u32x4 (&pk)[NP], int i) {
     const int ks = i / DT, dt = i % DT;
-    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-        __builtin_bit_cast(bf16x8, u32x4{vlo[i][0], vlo[i][1], vhi[i][0], vhi[i][1]}), __builtin_bit_cast(bf16x8, pk[ks]),
-        o[dt], 0, 0, 0);
+    const bf16x8 v = __builtin_bit_cast(bf16x8, u32x4{vlo[i][0], vlo[i][1], vhi[i][0], vhi[i][1]});
+    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, __builtin_bit_cast(bf16x8, pk[ks]), o[dt], 0, 0, 0);
+    if constexpr (PAIR)
+      o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, __builtin_bit_cast(bf16x8, pk[2 * TT + ks]), o[dt], 0, 0, 0);
   };
   // Step i (of 16) of a stage's exponentials: 2 TT scores, rounded to bf16 (the PV operand) and summed
-  // as rounded.  At one score pair per two steps the second exponential waits for the odd step.
+  // as rounded (PAIR: kept as a pair, summed in fp32).  At one score pair per two steps the second
+  // exponential waits for the odd step.
   float e_held = 0.f, x_held = 0.f;
-  auto exps = [&](const f32x16 (&s)[TT], u32x4 (&pk)[2 * TT], int i) {
+  auto exps = [&](const f32x16 (&s)[TT], u32x4 (&pk)[NP], int i) {
     const int pr = TT == 2 ? i : i >> 1;  // score pair
     const int u = pr >> 3, e = 2 * (pr & 7);
     if (TT == 2 || (i & 1) == 0) {
@@ -479,8 +494,17 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
       x_held = fmaf(s[u][e + 1], p.scale_log2, neg_m);
     }
     if (TT == 2 || (i & 1) == 1) {
-      uint32_t pair = pack_bf16x2(e_held, fast_exp2(x_held));
-      l_run = pf::add_pair(pair, l_run);
+      const float e1 = fast_exp2(x_held);
+      uint32_t pair;
+      if constexpr (PAIR) {
+        l_run += e_held + e1;
+        uint32_t rest = pf::split_pair(e_held, e1, pair);
+        pf::pin(rest);
+        pk[2 * TT + (pr >> 2)][pr & 3] = rest;
+      } else {
+        pair = pack_bf16x2(e_held, e1);
+        l_run = pf::add_pair(pair, l_run);
+      }
       pf::pin(pair);
       pk[pr >> 2][pr & 3] = pair;
     }
@@ -495,7 +519,7 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
   // Iteration t on the scores s (stage t) and the probabilities pp (stage t - 1): see the top of the
   // file.  The next scores go to sn (the last iteration's are of nothing and unused), stage t's
   // probabilities to pn.
-  auto iterate = [&](int t, f32x16 (&s)[TT], f32x16 (&sn)[TT], const u32x4 (&pp)[2 * TT], u32x4 (&pn)[2 * TT]) {
+  auto iterate = [&](int t, f32x16 (&s)[TT], f32x16 (&sn)[TT], const u32x4 (&pp)[NP], u32x4 (&pn)[NP]) {
     // K of stage t + 2 and V of stage t - 1 landed (the last kLead - 1 iterations' copies may be in flight),
     // this wave's own reads done
     pf::wait_vm<2 * kCopies * (kLead - 1), true>();
@@ -588,9 +612,9 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
     // The scores and probabilities alternate between two register sets, so the iterations go in pairs;
     // an odd count does stage 0 by itself.
     f32x16 s0[TT], s1[TT];
-    u32x4 p0[2 * TT], p1[2 * TT];
+    u32x4 p0[NP], p1[NP];
 #pragma unroll
-    for (int ks = 0; ks < 2 * TT; ++ks) p0[ks] = p1[ks] = u32x4{0u, 0u, 0u, 0u};
+    for (int ks = 0; ks < NP; ++ks) p0[ks] = p1[ks] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < 8; ++i) read_k(i);
     next_k();

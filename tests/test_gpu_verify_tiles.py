@@ -1,9 +1,8 @@
 """Speculative verify on prefill_tile_kernel's two-wave form: 17 to 64 query rows per KV head, with the
 new rows appended by the ranges that cover them (a chunk that straddles two stages or two ranges, empty
 caches, new rows on a page boundary), ragged batches whose ranges differ in number, the largest batch of
-the rule and the one past it, and the head counts and dims that the balanced kernel keeps because it is
-more exact there.  Caches bit-exact, outputs against the fp64 oracle, and against the
-balanced kernel the merge flag selects."""
+the rule and the one past it, and the head counts and dims that the balanced kernel keeps.  Caches
+bit-exact, outputs against the fp64 oracle, and against the balanced kernel the merge flag selects."""
 import numpy as np
 import pytest
 import torch
@@ -67,8 +66,8 @@ def test_verify_matches_oracle_and_balanced_kernel(gpu, case, append):
 
 @pytest.mark.parametrize("hd,nh,nk", [(64, 14, 2), (64, 16, 4), (128, 7, 1), (128, 14, 2)])
 def test_verify_keeps_the_more_exact_kernel(gpu, hd, nh, nk):
-    """Where the balanced kernel holds P as a bf16 pair (head_dim 64) or a maximum per phase (one or two
-    KV heads), the call is its launch: bit-identical to the one a merge flag selects."""
+    """head_dim 64 and one or two KV heads: the call is the balanced kernel's launch, bit-identical to the
+    one a merge flag selects."""
     cpu, d = make_paged_case(gpu, batch=6, ctx=[0, 27, 30, 253, 254, 600], page_size=256, n_kv=nk, n_heads=nh,
                              head_dim=hd, s_q=5, seed=5)
     kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, shared_prefix_tokens=0)
@@ -84,3 +83,33 @@ def test_verify_noalloc_is_bit_identical(gpu):
     a = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], **kw)
     b = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], noalloc=True, **kw)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("nh,nk,s_q,ctx", [(28, 4, 5, [600, 90, 1400, 33]), (40, 8, 6, [500, 150]),
+                                           (28, 4, 6, [16, 300, 45, 8, 120, 700])])
+def test_verify_error_is_the_output_rounding(gpu, nh, nk, s_q, ctx):
+    """Rounding N(0, s) values to bf16 leaves a relative error of 1.66e-3 (2-norm); P rounded to bf16 once
+    brings it to 1.9e-3 and more, held as a pair it adds nothing that shows."""
+    cpu, d = make_paged_case(gpu, batch=len(ctx), ctx=ctx, page_size=256, n_kv=nk, n_heads=nh, head_dim=128, s_q=s_q,
+                             seed=nh + s_q)
+    out = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], causal=True,
+                                            cache_seqlens=d["cache_seqlens"], block_table=d["block_table"])
+    ref, _, _ = pa.flash_attn_with_kvcache_ref(cpu["q"], cpu["k_cache"], cpu["v_cache"], cpu["k"], cpu["v"],
+                                               cache_seqlens=cpu["cache_seqlens"], block_table=cpu["block_table"],
+                                               causal=True)
+    got = out.double().cpu().numpy()
+    assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 1.8e-3
+
+
+def test_verify_infinite_value_stays_infinite(gpu):
+    """One infinite V element that every row sees: that output element is the infinity, the others finite
+    (neither half of P may meet it as a zero, or with the other sign)."""
+    cpu, d = make_paged_case(gpu, batch=2, ctx=[300, 40], page_size=256, n_kv=4, n_heads=28, head_dim=128, s_q=5,
+                             seed=2)
+    for b, value in ((0, float("inf")), (1, -float("inf"))):
+        d["v_cache"][int(cpu["block_table"][b, 0]), 7, 1, 3] = value
+    out = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], causal=True,
+                                            cache_seqlens=d["cache_seqlens"], block_table=d["block_table"])
+    assert (out[0, :, 7:14, 3] == float("inf")).all() and (out[1, :, 7:14, 3] == -float("inf")).all()
+    out[:, :, 7:14, 3] = 0
+    assert out.isfinite().all()
