@@ -264,7 +264,10 @@ int pkv_prefill_attn(const void* q, int64_t q_sb, int64_t q_ss, int64_t q_sh,
  * onto a long cached prefix, cuts every block's keys into ranges, keeps each range's unnormalised
  * output, row maximum and row sum in fp32 there and merges them in a second launch.  Same results
  * up to the order of fp32 sums.  pkv_prefill_workspace_bytes() is what such a call needs, 0 where
- * the keys are not split; workspace NULL never splits.  The same rules as pkv_decode_attn's
+ * the keys are not split; workspace NULL never splits.  The number of ranges follows from the sizes,
+ * max_blocks among them, so a wider block table may change the order of the sums; and it takes the
+ * table to be no wider than the longest sequence needs: over short sequences in a wide table the
+ * ranges cost a launch and save nothing.  The same rules as pkv_decode_attn's
  * workspace (the two may share one: the leading 64 KiB of counters are not touched).
  */
 size_t pkv_prefill_workspace_bytes(int32_t batch, int32_t s_q, int32_t n_heads, int32_t n_kv,

@@ -244,10 +244,16 @@ def _workspace(device: torch.device, nbytes: int, stream: int, allow_static: boo
         return ws
 
 
-def _prefill_workspace(device: torch.device, stream: int, *sizes: int) -> torch.Tensor | None:
+def _prefill_workspace(device: torch.device, stream: int, num_pages: int, *sizes: int) -> torch.Tensor | None:
     """The workspace of a prefill call that splits its keys, None where it does not: one per (device,
     stream), grow-only, and never handed to a capture.  A captured prefill does not split, because its
-    replays may run on any stream, beside eager calls that own the workspace."""
+    replays may run on any stream, beside eager calls that own the workspace.
+
+    The library splits by the block table's width (sizes[-1] columns).  A table as wide as the pool
+    (DecodeBatch's) says nothing of the lengths, so such a call does not split: over short sequences the
+    ranges would cost it 3 to 14 us (17 us a call at 128 keys) and save nothing."""
+    if sizes[-1] >= num_pages:
+        return None
     nbytes = _prefill_bytes(*sizes)
     if nbytes == 0 or torch.cuda.is_current_stream_capturing():
         return None
@@ -542,10 +548,10 @@ def flash_attn_with_kvcache(
             st.data_ptr(), stream)
         _lib.check(rc, "pkv_decode_attn")
     else:
-        # a table of fewer than 16 stages of 32 keys never splits: short prompts are host-bound (18 us a
-        # call), and asking the library costs them 0.3 us
-        ws = None if noalloc or max_blocks * page_size < 512 else \
-            _prefill_workspace(device, stream, batch, s_q, n_heads, n_kv, hd, page_size, max_blocks)
+        # a table whose longest sequence may hold fewer than 24 stages of 32 keys never splits: short prompts
+        # are host-bound (17 us a call), and asking the library costs them 0.3 us
+        ws = None if noalloc or (max_blocks - 1) * page_size < 736 else \
+            _prefill_workspace(device, stream, num_pages, batch, s_q, n_heads, n_kv, hd, page_size, max_blocks)
         if ws is None:
             rc = lib.pkv_prefill_attn(
                 q.data_ptr(), *qs, kp, *ks, vp, *vs,
@@ -667,7 +673,7 @@ def prefill_attention(q, k_cache, v_cache, k=None, v=None, *, cache_seqlens, blo
     scale = float(softmax_scale) if softmax_scale is not None else 1.0 / math.sqrt(hd)
     lib = _lib.load()
     stream = _stream_ptr(q.device)
-    ws = _prefill_workspace(k_cache.device, stream, batch, s_q, n_heads, n_kv, hd, page_size, block_table.shape[1])
+    ws = _prefill_workspace(k_cache.device, stream, num_pages, batch, s_q, n_heads, n_kv, hd, page_size, block_table.shape[1])
     rc = lib.pkv_prefill_attn_ws(
         q.data_ptr(), *qs, kp, *ks, vp, *vs,
         k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),

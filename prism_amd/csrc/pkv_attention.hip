@@ -3055,18 +3055,34 @@ static void launch_decode_hd(const AttnParams& p, int batch, hipStream_t stream)
 constexpr int kPrefillNT = 2;
 constexpr int kPrefillW = 4;
 
-// Key ranges per item of a prefill launch: as many as keep the workgroups within one round of two per
-// CU, no more than the block table has ranges of kMinStages for.  1 where the row blocks fill half the
-// card by themselves, and where no sequence can hold kSplitStages: a workgroup alone on its CU takes
-// 0.5-0.6 us per stage, and the ranges add a second launch of about 4 us.
+// Key ranges per item of a prefill launch, 1 where splitting does not pay.  What is known of the keys is
+// the block table's width, taken as no wider than its longest sequence needs: then that sequence has at
+// least n stages.  Ranges hold at least kMinStages; their number is what one round of one workgroup per
+// CU has room for, or of two where one would be fewer than four ranges or each would still be deep.
+// Splitting saves stages on the longest item's chain, of `stage` us each; it adds a launch (2.5 us with
+// the host's share) and the fp32 partials, written and read back: up to `fill` us at one workgroup per
+// CU and above.  Two workgroups on a CU slow each other (0.75 us a stage at 352 workgroups, 0.96 at 512).
+// A call below `floor` us is the host's time either way, 17 us unsplit and 20.5 split.
+// us a call, unsplit / split, by items and stages (head_dim 128):
+//    24 items: n = 20 20.5 / 21.1, 24 22.5 / 21.2, 48 34.5 / 21.8, 128 74.8 / 27.4
+//    44: n = 20 20.4 / 21.7, 24 22.5 / 22.0, 48 34.5 / 25.4     64: n = 24 22.8 / 24.3, 32 26.7 / 26.1
+//   128: n = 40 31.3 / 33.1, 48 35.3 / 34.6                    256: n = 128 81.9 / 86.6, 256 152 / 148
+// and with stages of 64 (head_dim 64), 88 items: n = 16 20.1 / 23.3, 24 25.5 / 24.8, 64 53.0 / 30.8.
 static int prefill_splits(int batch, int64_t R, int n_kv, int head_dim, int page_size, int max_blocks) {
   const int tok = head_dim == 128 ? pf::Geo<128>::TOK : pf::Geo<64>::TOK;
   if (page_size < tok) return 1;
+  const double stage = head_dim == 128 ? 0.51 : 0.68, fill = head_dim == 128 ? 9.7 : 5.4, floor = 21.3;
+  const int64_t cus = device_cu_count();
   const int64_t items = (R + pf::kRows - 1) / pf::kRows * n_kv * batch;
-  const int64_t by_grid = 2 * int64_t(device_cu_count()) / items;
-  const int64_t by_keys = int64_t(max_blocks) * page_size / (tok * pf::kMinStages);
-  const int64_t s = by_grid < by_keys ? by_grid : by_keys;
-  return s < 2 || by_keys * pf::kMinStages < pf::kSplitStages ? 1 : int(s);
+  const int64_t n = int64_t(max_blocks - 1) * page_size / tok + 1;
+  const int64_t one = cus / items, two = 2 * cus / items;
+  int64_t s = one >= 4 && n < pf::kDeepStages * two ? one : two;
+  s = s < n / pf::kMinStages ? s : n / pf::kMinStages;
+  if (s < 2 || 9.5 + stage * double(n) < floor) return 1;
+  const double per_cu = double(items * s) / double(cus);
+  const double slow = per_cu > 1 ? 0.7 + 0.55 * per_cu : 1;
+  const double saved = stage * (double(n) - double((n + s - 1) / s) * slow);
+  return saved > 2.5 + fill * (per_cu < 1 ? per_cu : 1) ? int(s) : 1;
 }
 static size_t ws_bytes_prefill(int batch, int64_t R, int n_kv, int head_dim, int splits) {
   if (splits < 2) return 0;

@@ -77,14 +77,15 @@ enum Dest {
   kSplit,    // one of max_splits key ranges: fp32 O and (m, l) for prefill_merge_kernel
 };
 
-// Key ranges.  A call with few row blocks (150 tokens onto 3500 at the 7B shape: 36 workgroups of 115
-// stages) leaves most CUs idle at 0.6 us per stage; cut into 14 ranges each, it takes 30 us a call
-// instead of 70, the merge launch included.  The partials stay fp32.
+// Key ranges.  A call with few row blocks (150 tokens onto 3500 at the 7B shape: 36 items of 115 stages)
+// leaves most CUs idle at 0.5 us per stage; cut into ranges it takes 28 us a call instead of 68, the merge
+// launch included.  The partials stay fp32.
 // Key ranges of an item of n stages in a kSplit launch: `chunk` stages each, at least kMinStages (a
-// range pays about two stages' time to start and one to end).  One range writes its rows directly.
-constexpr int kMinStages = 4;
+// range pays about two stages' time to start and one to end, and a partial of 66 KB: 3 ranges of 8 are
+// as fast as 6 of 4 at 24 items and faster from 44 on).  One range writes its rows directly.
+constexpr int kMinStages = 8;
 constexpr int kMinVerifyStages = 5;
-constexpr int kSplitStages = 16;  // stages a sequence must be able to hold for a kSplit launch
+constexpr int kDeepStages = 12;  // two workgroups per CU from this many stages a range on
 struct Ranges {
   int chunk, count;
 };

@@ -123,6 +123,24 @@ def test_prefill_workspace_bytes_of_rejected_sizes_is_zero(lib, sizes):
     assert lib.pkv_prefill_workspace_bytes(*sizes) == 0
 
 
+@pytest.mark.parametrize("sizes,splits", [
+    # (batch, s_q, n_heads, n_kv, head_dim, page_size, max_blocks), splits with 256 CUs.  A table of m pages
+    # stands for a sequence that reaches its last page: (m - 1) pages and a key
+    ((1, 45, 28, 4, 128, 256, 2), 1), ((1, 45, 28, 4, 128, 256, 3), 1), ((1, 45, 28, 4, 128, 256, 4), 3),
+    ((4, 100, 28, 4, 128, 256, 5), 1), ((4, 100, 28, 4, 128, 256, 9), 5),     # 96 items
+    ((4, 200, 28, 4, 128, 256, 9), 1), ((4, 200, 28, 4, 128, 256, 16), 2),    # 176 items
+    ((4, 200, 40, 8, 128, 256, 17), 1), ((4, 400, 40, 8, 128, 256, 64), 1),   # 256 and 512 items
+    ((1, 150, 28, 4, 128, 256, 15), 7), ((1, 150, 28, 4, 128, 256, 64), 14),  # 36: one round, then two
+    ((1, 45, 14, 2, 64, 256, 4), 1), ((1, 45, 14, 2, 64, 256, 6), 2), ((4, 400, 14, 2, 64, 256, 8), 1),
+    ((1, 150, 28, 4, 128, 4096, 1), 1), ((1, 150, 28, 4, 128, 16, 200), 1),   # one page; pages below a stage
+])
+def test_prefill_splits_where_ranges_pay(lib, sizes, splits):
+    batch, s_q, nh, nkv, hd, page, mb = sizes
+    items = -(-s_q * (nh // nkv) // 128) * nkv * batch
+    want = 0 if splits == 1 else 65536 + items * splits * 128 * (hd + 2) * 4
+    assert lib.pkv_prefill_workspace_bytes(*sizes) == want
+
+
 def test_copy_and_gather_argument_errors(lib):
     rc = lib.pkv_copy_pages(A16, A16, 2, A16, A16, None, 3, 1000, 1 << 18, 1024, 256, 10, 10, None, None)
     assert rc == _lib.PKV_EINVAL and "pkv_copy_pages" in lib.pkv_last_error().decode()

@@ -318,7 +318,7 @@ def test_a_capture_never_borrows_a_prefill_workspace(monkeypatch):
     capturing = [False]
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
     dev, A, B, C = torch.device("cpu", 0), 11, 22, 33
-    sizes = (1, 150, 28, 4, 128, 256, 15)  # 150 tokens onto 3500 at the 7B shape
+    sizes = (20, 1, 150, 28, 4, 128, 256, 15)  # a pool of 20 pages; 150 tokens onto 3500 at the 7B shape
     pre = attn._prefill_workspace(dev, B, *sizes)
     pre_a = attn._prefill_workspace(dev, A, *sizes)
     dec = attn._workspace(dev, 2 << 20, A)
@@ -331,10 +331,18 @@ def test_a_capture_never_borrows_a_prefill_workspace(monkeypatch):
     assert attn._prefill_workspace(dev, A, *sizes).data_ptr() == pre_a.data_ptr() != got.data_ptr()
 
 
+def test_a_table_as_wide_as_the_pool_does_not_split(monkeypatch):
+    monkeypatch.setattr(attn, "_prefill_workspaces", {})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    dev, sizes = torch.device("cpu", 0), (1, 150, 28, 4, 128, 256, 64)
+    assert attn._prefill_workspace(dev, 1, 64, *sizes) is None
+    assert attn._prefill_workspace(dev, 1, 65, *sizes) is not None
+
+
 def test_a_prefill_without_memory_for_its_workspace_runs_unsplit(monkeypatch):
     monkeypatch.setattr(attn, "_prefill_workspaces", {})
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
-    dev, sizes = torch.device("cpu", 0), (1, 150, 28, 4, 128, 256, 15)
+    dev, sizes = torch.device("cpu", 0), (20, 1, 150, 28, 4, 128, 256, 15)
 
     def full(*a, **k):
         raise torch.OutOfMemoryError("no memory")
