@@ -245,9 +245,10 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const NormParams p) {
 
 // ---------------------------------------------------------------------------------------------
 // SiLU(gate) * up over rows of m values: out = bf16(bf16(silu(g)) * u), the two roundings of the
-// reference's F.silu(gu[..., :m]) * gu[..., m:] on bf16 tensors.  Grid (256 16-byte chunks of a row,
-// rows).  Memory bounds it: 4096 x 13824 is 340 MB in 58 us (5.9 TB/s).  A 64-bit division per chunk to
-// find the row and eight IEEE divisions held it at 60.
+// reference's F.silu(gu[..., :m]) * gu[..., m:] on bf16 tensors.  One 16-byte chunk per thread, counted
+// over the rows, so that narrow rows fill their waves (a grid row per tensor row took 137 us where m = 64
+// moves 200 MB in 31).  Memory bounds it: 4096 x 13824 is 340 MB in 58 us (5.9 TB/s).  A 64-bit
+// division per chunk to find the row and eight IEEE divisions held it at 60.
 //
 // STREAM reads gate and up non-temporally, for launches that read more than the eight 4 MiB L2s hold
 // (kStreamBytes).  14B, plain / non-temporal: right behind the launch that wrote them, 2048 rows 25.2 /
@@ -262,8 +263,10 @@ struct SiluParams {
   int64_t u_stride;
   uint16_t* out;
   int64_t o_stride;
-  int64_t rows;
-  int m;
+  uint32_t chunks;      // of the launch, below 2^31
+  uint32_t row_chunks;
+  uint32_t magic;       // chunk i is in row (i magic) >> shift
+  int shift;
 };
 
 constexpr int64_t kStreamBytes = int64_t(32) << 20;
@@ -280,30 +283,30 @@ __device__ __forceinline__ float div_bounded(float g, float d) {
 
 template <bool STREAM>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const SiluParams p) {
-  const int c = int(blockIdx.x) * 256 + int(threadIdx.x);
-  if (c >= p.m / 8) return;
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= p.chunks) return;
+  const uint32_t r = uint32_t((uint64_t(i) * p.magic) >> p.shift);
+  const int64_t c = int64_t(i - r * p.row_chunks) * 8;
   auto load = [](const uint16_t* src) {
     return STREAM ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src)) : ld16(src);
   };
-  for (int64_t r = blockIdx.y; r < p.rows; r += gridDim.y) {
-    float gf[8], uf[8], s[8];
-    unpack8(load(p.gate + r * p.g_stride + 8 * c), gf);
-    unpack8(load(p.up + r * p.u_stride + 8 * c), uf);
-    float big = 0.f;
+  float gf[8], uf[8], s[8];
+  unpack8(load(p.gate + r * p.g_stride + c), gf);
+  unpack8(load(p.up + r * p.u_stride + c), uf);
+  float big = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) big = fmaxf(big, fabsf(gf[e]));
-    if (__builtin_expect(big < 80.f, 1)) {  // a NaN passes, and stays one
+  for (int e = 0; e < 8; ++e) big = fmaxf(big, fabsf(gf[e]));
+  if (__builtin_expect(big < 80.f, 1)) {  // a NaN passes, and stays one
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s[e] = div_bounded(gf[e], 1.f + __expf(-gf[e]));
-    } else {
+    for (int e = 0; e < 8; ++e) s[e] = div_bounded(gf[e], 1.f + __expf(-gf[e]));
+  } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s[e] = gf[e] / (1.f + __expf(-gf[e]));
-    }
-    unpack8(pack8(s), s);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s[e] *= uf[e];
-    __builtin_nontemporal_store(pack8(s), reinterpret_cast<u32x4*>(p.out + r * p.o_stride + 8 * c));
+    for (int e = 0; e < 8; ++e) s[e] = gf[e] / (1.f + __expf(-gf[e]));
   }
+  unpack8(pack8(s), s);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) s[e] *= uf[e];
+  __builtin_nontemporal_store(pack8(s), reinterpret_cast<u32x4*>(p.out + r * p.o_stride + c));
 }
 
 }  // namespace pkv
@@ -422,17 +425,25 @@ extern "C" int pkv_silu_mul(const void* gate, int64_t g_stride, const void* up, 
     return fail(PKV_EINVAL, "%s: rows must be 16-byte aligned", fn);
   const int64_t total = rows * (m / 8);
   if (total == 0) return PKV_OK;
-  SiluParams p;
-  p.gate = static_cast<const uint16_t*>(gate);
-  p.g_stride = g_stride;
-  p.up = static_cast<const uint16_t*>(up);
-  p.u_stride = u_stride;
-  p.out = static_cast<uint16_t*>(out);
-  p.o_stride = o_stride;
-  p.rows = rows;
-  p.m = m;
-  const dim3 grid(unsigned((m / 8 + 255) / 256), unsigned(rows < 65535 ? rows : 65535));
   auto* kernel = total * 32 > kStreamBytes ? silu_mul_kernel<true> : silu_mul_kernel<false>;
-  kernel<<<grid, 256, 0, static_cast<hipStream_t>(stream)>>>(p);
+  SiluParams p;
+  p.g_stride = g_stride;
+  p.u_stride = u_stride;
+  p.o_stride = o_stride;
+  p.row_chunks = uint32_t(m / 8);
+  // i / d for i < 2^31, with 2^l the power of two at or above d: magic = floor(2^(31 + l) / d) + 1 fits in
+  // 32 bits, and magic d exceeds 2^(31 + l) by at most d <= 2^l, so i times the excess stays below 2^(31 + l)
+  const int l = ilog2(p.row_chunks);
+  p.magic = uint32_t((uint64_t(1) << (31 + l)) / p.row_chunks + 1);
+  p.shift = 31 + l;
+  const int64_t slab = 0x7fffffff / p.row_chunks;  // rows of a launch
+  for (int64_t r0 = 0; r0 < rows; r0 += slab) {
+    const int64_t n = rows - r0 < slab ? rows - r0 : slab;
+    p.gate = static_cast<const uint16_t*>(gate) + r0 * g_stride;
+    p.up = static_cast<const uint16_t*>(up) + r0 * u_stride;
+    p.out = static_cast<uint16_t*>(out) + r0 * o_stride;
+    p.chunks = uint32_t(n) * p.row_chunks;
+    kernel<<<(p.chunks + 255) / 256, 256, 0, static_cast<hipStream_t>(stream)>>>(p);
+  }
   return check_launch(fn);
 }

@@ -235,3 +235,31 @@ def test_silu_mul_infinities_and_nan(gpu):
     zero = torch.tensor([[0.0, -0.0] * 4], dtype=torch.bfloat16, device=gpu)
     out = prism_amd.silu_mul(zero, torch.ones_like(zero))
     assert torch.equal(out.signbit(), zero.signbit()) and (out == 0).all()
+
+
+@pytest.mark.parametrize("rows,m", [(4097, 24), (300, 520), (257, 2056), (5, 16392), (70000, 16)])
+def test_silu_mul_rows_packed_into_waves(gpu, rows, m):
+    """Workgroups that begin and end inside a row, over several rows or within one, strided."""
+    buf = _rand((rows, 2 * m + 16), rows + m, 2.0)
+    ref = ep.silu_mul_ref(buf[:, :m].float().numpy(), buf[:, m + 8:2 * m + 8].float().numpy())
+    d = buf.to(gpu)
+    _ulp_close(prism_amd.silu_mul(d[:, :m], d[:, m + 8:2 * m + 8]), ref, f"silu_mul {rows}x{m}", 1.0)
+
+
+def test_silu_mul_time_does_not_depend_on_the_row_width(gpu):
+    """The same 8 Mi values as rows of 8 and as rows of 2048: the same bytes, so no multiple of the time
+    (27 times it, with a workgroup per row)."""
+    def us(rows, m):
+        gu = torch.zeros(rows, 2 * m, dtype=torch.bfloat16, device=gpu)
+        best = float("inf")
+        for _ in range(10):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                prism_amd.silu_mul(gu[:, :m], gu[:, m:])
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 100)
+        return best
+
+    assert us(1 << 20, 8) < 4 * us(4096, 2048)
