@@ -268,34 +268,6 @@ __device__ __forceinline__ void load_q(const AttnParams& p, const SeqView& sv, i
   }
 }
 
-// load_q for the cascade prefix pass: rows r < batch * R of the whole batch (sequence r / R,
-// row r % R of it), every one seeing keys [0, last_key].
-template <int HD, int NT>
-__device__ __forceinline__ void load_q_batch_rows(const AttnParams& p, int h, int row0, int last_key,
-                                                  bf16x8 (&qf)[NT][HD / 32], int (&lim)[NT]) {
-  const int lane = threadIdx.x & 63;
-  const int li = lane & 15;
-  const int lq = lane >> 4;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int ra = row0 + li + 16 * nt;
-    if (ra < p.batch * p.R) {
-      const int b = ra / p.R;
-      const int rr = ra - b * p.R;
-      const int j = rr / p.g;
-      const int hq = rr - j * p.g;
-      const uint16_t* base = p.q + b * p.q_sb + j * p.q_ss + (h * p.g + hq) * p.q_sh + 8 * lq;
-#pragma unroll
-      for (int kk = 0; kk < HD / 32; ++kk) qf[nt][kk] = __builtin_bit_cast(bf16x8, ld16(base + 32 * kk));
-      lim[nt] = last_key;
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < HD / 32; ++kk) qf[nt][kk] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-      lim[nt] = kNoQueryRow;
-    }
-  }
-}
-
 // A pointer the whole wave agrees on, pinned to scalar registers.
 template <typename T>
 __device__ __forceinline__ T* uniform_ptr(T* ptr) {
@@ -3122,6 +3094,7 @@ static size_t ws_bytes_verify(int batch, int n_kv, int head_dim) {
 static bool use_verify_tiles(int batch, int n_kv, int head_dim, int R, int page_size, bool lean, int32_t flags) {
   return lean && lean_geom(head_dim, n_kv) == kGeom128x4 && R > 16 && page_size >= pf::Geo<128>::TOK &&
          (flags & ~PKV_DECODE_RESET_COUNTERS) == 0 && int64_t(batch) * n_kv <= device_cu_count() &&
+         batch <= pf::kVerifyBatch &&
          ws_bytes_verify(batch, n_kv, head_dim) <= kScratchBytes;
 }
 static void launch_verify_tiles(const AttnParams& p, int batch, hipStream_t stream) {

@@ -151,9 +151,9 @@ __device__ __forceinline__ void pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
 // one sequence: a ragged batch keeps every workgroup at the same work, whatever the longest sequence.
 // Range w of KV head h is workgroup w n_kv + h, so that each XCD's L2 serves few heads (a cached prefix
 // that the batch shares is then read once per XCD and head).
-constexpr int kVerifyBatch = 256;
+constexpr int kVerifyBatch = 64;  // one sequence per lane
 struct VerifyPlan {
-  int n[kVerifyBatch / 64];  // stages of sequence 64 i + lane (0 past the batch)
+  int n;  // stages of sequence `lane` (0 past the batch)
   int chunk;
 };
 template <int TOK>
@@ -161,43 +161,20 @@ __device__ __forceinline__ VerifyPlan verify_plan(const AttnParams& p) {
   const int lane = threadIdx.x & 63;
   const int cap = p.max_blocks << p.log2_page;
   VerifyPlan v;
-#pragma unroll
-  for (int i = 0; i < kVerifyBatch / 64; ++i) {
-    v.n[i] = 0;
-    if (64 * i < p.batch && 64 * i + lane < p.batch) {
-      const int c = min(max(p.seqlens[64 * i + lane], 0), cap);  // as seq_lengths clamps it
-      v.n[i] = max(stages_of<TOK>(p, min(c + (p.has_new ? p.s_q : 0), cap), p.R - 1), 1);
-    }
+  v.n = 0;
+  if (lane < p.batch) {
+    const int c = min(max(p.seqlens[lane], 0), cap);  // as seq_lengths clamps it
+    v.n = max(stages_of<TOK>(p, min(c + (p.has_new ? p.s_q : 0), cap), p.R - 1), 1);
   }
-  int total = 0;
-#pragma unroll
-  for (int i = 0; i < kVerifyBatch / 64; ++i)
-    if (64 * i < p.batch) total += __builtin_amdgcn_readlane(wave_incl_scan(v.n[i]), 63);
+  const int total = __builtin_amdgcn_readlane(wave_incl_scan(v.n), 63);
   v.chunk = max((total + p.lean_grid - 1) / p.lean_grid, kMinVerifyStages);
   // every sequence's last range may be short: lengthen the ranges until they fit one round
   for (int tries = 0; tries < 16; ++tries) {
-    int ranges = 0;
-#pragma unroll
-    for (int i = 0; i < kVerifyBatch / 64; ++i)
-      if (64 * i < p.batch) ranges += __builtin_amdgcn_readlane(wave_incl_scan((v.n[i] + v.chunk - 1) / v.chunk), 63);
+    const int ranges = __builtin_amdgcn_readlane(wave_incl_scan((v.n + v.chunk - 1) / v.chunk), 63);
     if (ranges <= max(p.lean_grid, p.batch)) break;
     v.chunk += max(v.chunk / 16, 1);
   }
   return v;
-}
-// Calls f(i, ranges of sequence 64 i + lane, their inclusive sum inside the 64, ranges before the 64).
-template <typename F>
-__device__ __forceinline__ void verify_ranges(const AttnParams& p, const VerifyPlan& v, F&& f) {
-  int base = 0;
-#pragma unroll
-  for (int i = 0; i < kVerifyBatch / 64; ++i) {
-    if (64 * i < p.batch) {
-      const int r = (v.n[i] + v.chunk - 1) / v.chunk;
-      const int incl = wave_incl_scan(r);
-      f(i, r, incl, base);
-      base += __builtin_amdgcn_readlane(incl, 63);
-    }
-  }
 }
 
 }  // namespace pf
@@ -258,17 +235,13 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
       const int w = i / p.n_kv;
       const pf::VerifyPlan v = pf::verify_plan<TOK>(p);
       chunk = v.chunk;
-      b = -1;
-      pf::verify_ranges(p, v, [&](int k, int r, int incl, int base) {
-        const uint64_t hit = __ballot(base + incl > w);
-        if (b < 0 && hit) {
-          const int first = int(__builtin_ctzll(hit));
-          b = 64 * k + first;
-          count = __builtin_amdgcn_readlane(r, first);
-          split = w - base - (__builtin_amdgcn_readlane(incl, first) - count);
-        }
-      });
-      if (b < 0) return;  // fewer ranges than the grid allows for
+      const int ranges = (v.n + chunk - 1) / chunk;
+      const int incl = wave_incl_scan(ranges);
+      const uint64_t hit = __ballot(incl > w);
+      if (!hit) return;  // fewer ranges than the grid allows for
+      b = int(__builtin_ctzll(hit));
+      count = __builtin_amdgcn_readlane(ranges, b);
+      split = w - (__builtin_amdgcn_readlane(incl, b) - count);
       // for the merge: where the sequence's ranges start, and how many they are
       if (h == 0 && split == 0 && threadIdx.x == 0) {
         p.ws_cnt[2 * b] = w;
