@@ -619,11 +619,13 @@ def tile_stamps_bench(args, dev) -> dict:
         w = getattr(workloads, args.stamps_of)(dev, seed=args.seed)
     kv, L = w.kv, w.layers
     outs = [torch.empty_like(q) for q in w.q]
+    # verify runs the prefill tile kernel, which has no stamps, unless a merge is asked for
+    two_pass = True if w.s_q > 1 else None
 
     def call(l):
         prism_amd.flash_attn_with_kvcache(w.q[l], kv.k_caches[l], kv.v_caches[l], k=w.k[l], v=w.v[l],
                                           cache_seqlens=w.cache_seqlens, block_table=w.block_table, causal=True,
-                                          out=outs[l])
+                                          two_pass=two_pass, out=outs[l])
 
     def step():
         for l in range(L):
@@ -680,8 +682,8 @@ def tile_stamps_bench(args, dev) -> dict:
                          "merge_done": us(m[mu, 2].max()) if len(mu) else None,
                          "last_arrival": max((r["arrival"] for r in rows if r["arrival"] is not None), default=None)})
 
-    def med(xs):
-        return round(float(np.median(xs)), 2)
+    def med(xs):  # None without samples: a verify launch has no in-launch merges
+        return round(float(np.median(xs)), 2) if xs else None
 
     def pct(xs, q):
         return round(float(np.percentile(xs, q)), 2)
@@ -1020,8 +1022,8 @@ def main() -> int:
                 "frac": round(gbs_unique / HBM_PEAK_GBS, 4), "traffic": traffic,
                 **({"traffic_source": traffic_src} if traffic_src else {}),
                 "mfma_tflops": round(tflops, 2), "mfma_frac": round(tflops / MFMA_BF16_PEAK_TFLOPS, 4),
-                "kernel": "one pkv_decode_attn call (s_q=5, 35 query rows per KV head) = decode_lean_kernel<3> "
-                          "(balanced tile ranges, 3 MFMA row tiles per wave) + combine_lean_kernel; bytes count "
+                "kernel": "one pkv_decode_attn call (s_q=5, 35 query rows per KV head) = prefill_tile_kernel<128, 2, 2> "
+                          "(key ranges, two waves of 32 query rows, append) + prefill_merge_kernel; bytes count "
                           "every key once, the shared prefix once for the batch; " + per_call,
                 "bytes_per_call": unique_layer, "flops_per_call": flops_layer, "avg_call_us": round(call_us, 3),
                 "per_sequence_bytes_per_call": bytes_layer, "gbs_per_sequence": round(gbs, 1),

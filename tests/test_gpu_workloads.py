@@ -250,3 +250,15 @@ def test_config5_prefix_cow_verify_compaction_transfer(gpu):
     chk.check(out, "config5 verify after compaction, layer 13")
     del chk, w
     _free()
+
+
+def test_tile_stamps_of_a_verify_batch(gpu):
+    # bench.py --workload tile-stamps --stamps-of config5: the stamped kernel is the one that runs
+    import argparse
+
+    import bench
+
+    args = argparse.Namespace(stamps_of="config5", seed=0, batch=0, stamp_calls=2, steps=2, warmup=1)
+    res = bench.tile_stamps_bench(args, gpu)
+    assert res["grid"] > 0 and res["tiles"] > 0 and res["calls"] == 2
+    _free()
