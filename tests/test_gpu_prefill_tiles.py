@@ -147,3 +147,18 @@ def test_prefill_captured_runs_unsplit(gpu):
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(out2, want)
         assert torch.equal(prism_amd.flash_attn_with_kvcache(*args, **kw), split)
+
+
+@pytest.mark.parametrize("hd,page,ctx", [(128, 32, [4200, 4500]), (64, 64, [8300, 9000])])
+def test_prefill_block_table_window_refills(gpu, hd, page, ctx):
+    """Over 130 pages in one workgroup's walk (unsplit): its 64-column window of the table is loaded twice more
+    inside the loop."""
+    cpu, d = make_paged_case(gpu, batch=2, ctx=ctx, page_size=page, n_kv=1, n_heads=7, head_dim=hd, s_q=20, seed=hd)
+    out = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], noalloc=True,
+                                            cache_seqlens=d["cache_seqlens"], block_table=d["block_table"],
+                                            causal=True)
+    ref, _, _ = pa.flash_attn_with_kvcache_ref(cpu["q"], cpu["k_cache"], cpu["v_cache"], cpu["k"], cpu["v"],
+                                               cache_seqlens=cpu["cache_seqlens"], block_table=cpu["block_table"],
+                                               causal=True)
+    assert_attn_close(out, ref, f"hd {hd}")
+    assert prism_amd.read_status(gpu) == 0

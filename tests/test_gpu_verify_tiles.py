@@ -9,7 +9,7 @@ import torch
 
 import prism_amd
 from oracle import paged_attention as pa
-from pkv_testutil import make_paged_case
+from pkv_testutil import assert_attn_close, make_paged_case
 
 pytestmark = pytest.mark.gpu
 
@@ -113,3 +113,35 @@ def test_verify_infinite_value_stays_infinite(gpu):
     assert (out[0, :, 7:14, 3] == float("inf")).all() and (out[1, :, 7:14, 3] == -float("inf")).all()
     out[:, :, 7:14, 3] = 0
     assert out.isfinite().all()
+
+
+@pytest.mark.parametrize("base,stride", [(8, 0), (0, 8), (8, 8)], ids=["base", "page-stride", "both"])
+def test_verify_appends_off_a_cache_line_keep_the_balanced_kernel(gpu, base, stride):
+    """Caches 16 bytes off a 128-byte line, or pages that are: a row appended in the launch could share a line
+    with one that another workgroup has read, so an appending call stays on the balanced kernel.  Without an
+    append it does not matter."""
+    P, nk = 64, 4
+    cpu, d = make_paged_case(gpu, batch=4, ctx=[0, 63, 130, 700], page_size=P, n_kv=nk, n_heads=28, head_dim=128,
+                             s_q=5, seed=4)
+
+    def view(t):
+        ps = t[0].numel() + stride
+        buf = torch.zeros(base + t.shape[0] * ps, dtype=t.dtype, device=gpu)
+        v = buf.as_strided(t.shape, (ps, nk * 128, 128, 1), base)
+        return v.copy_(t)
+
+    kc, vc = view(d["k_cache"]), view(d["v_cache"])
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, shared_prefix_tokens=0)
+    other = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"].clone(), d["v_cache"].clone(), d["k"], d["v"],
+                                              two_pass=True, **kw)
+    out = prism_amd.flash_attn_with_kvcache(d["q"], kc, vc, d["k"], d["v"], **kw)
+    ref, kb, vb = pa.flash_attn_with_kvcache_ref(cpu["q"], cpu["k_cache"], cpu["v_cache"], cpu["k"], cpu["v"],
+                                                 cache_seqlens=cpu["cache_seqlens"], block_table=cpu["block_table"],
+                                                 causal=True)
+    assert np.array_equal(pa.bf16_bits(kc), kb) and np.array_equal(pa.bf16_bits(vc), vb)
+    assert torch.equal(out, other)
+    assert_attn_close(out, ref, "off a cache line")
+    kw["cache_seqlens"] = d["cache_seqlens"] + 5
+    again = prism_amd.flash_attn_with_kvcache(d["q"], kc, vc, **kw)
+    assert_attn_close(again, ref, "off a cache line, no append")
+    assert prism_amd.read_status(gpu) == 0
