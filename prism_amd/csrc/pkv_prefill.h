@@ -193,6 +193,7 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
   using G = pf::Geo<HD>;
   constexpr int kRows = 32 * W;
   constexpr int kLead = W == pf::kWaves ? 3 : 2;  // iterations between a copy's issue and its use
+  static_assert(kLead == 2 || kLead == 3, "V copies start in iteration -2 or -1");
   constexpr int kRing = kLead + 1;                // slots of the K and of the V ring
   constexpr int kCopies = 8 / W;                  // copies of a K (or V) stage per wave
   constexpr int TT = G::TT, DT = G::DT, KK = G::KK, TOK = G::TOK;
@@ -366,13 +367,13 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
   char* const ring_k = lds;
   char* const ring_v = lds + kRing * G::STAGE;
   // Iteration t issues the copies of K stage t + kLead + 2 and V stage t + kLead - 1 (from t = -kLead -
-  // 2), kCopies of each per wave.  Those of a stage that does not exist are issued too, with an empty
-  // buffer: they fetch nothing and write zeros to a free slot, and the loop has neither branches nor
+  // 2, V from stage 0), kCopies of each per wave.  Those of a stage past the last are issued too, with an
+  // empty buffer: they fetch nothing and write zeros to a free slot, and the loop has neither branches nor
   // other counts to wait for.  A stage's page lookup serves its K copies and, three iterations later,
   // its V copies: off1 .. off3 hold the offsets of the stages in between, oldest first.
   int64_t off1 = 0, off2 = 0, off3 = 0;
-  int slot_k = 0, slot_v = (kRing * 2 - 3) % kRing * G::STAGE;  // ring slots the next copies go to (V from stage -3)
-  int left_k = n, left_v = n + 3;                               // stages left to copy
+  int slot_k = 0, slot_v = 0;    // ring slots the next copies go to
+  int left_k = n, left_v = n;    // stages left to copy
   auto next_slot = [](int slot) { return slot == (kRing - 1) * G::STAGE ? 0 : slot + G::STAGE; };
   auto next_stage = [&] {
     if (__builtin_expect((T_k & pmask) == 0 && left_k > 0, 0)) page_start();
@@ -394,7 +395,7 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
   // off_v: off1 as it was before this iteration's next_stage()
   auto copy_v = [&](int k, int64_t off_v) {
     const int i = wave + W * k;
-    pf::copy_1k(p.v_cache + off_v, left_v > 0 && left_v <= n ? TOK * row_bytes : 0, vv, i * G::RPC * row_bytes,
+    pf::copy_1k(p.v_cache + off_v, left_v > 0 ? TOK * row_bytes : 0, vv, i * G::RPC * row_bytes,
                 ring_v + slot_v + i * 1024);
     if (k == kCopies - 1) {
       slot_v = next_slot(slot_v);
@@ -570,17 +571,18 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
       for (int i = 0; i < kCopies; ++i) *reinterpret_cast<u32x4*>(z + i * 1024 * W) = u32x4{0u, 0u, 0u, 0u};
     }
     page_start();
-    auto copies = [&] {
-      const int64_t off_v = off1;
+    int64_t off_v = 0;
+    for (int t = -kLead - 2; t < -1; ++t) {
+      off_v = off1;
       next_stage();
 #pragma unroll
       for (int k = 0; k < kCopies; ++k) copy_k(k);
+    }
+    if (kLead == 3)
 #pragma unroll
       for (int k = 0; k < kCopies; ++k) copy_v(k, off_v);
-    };
-    for (int t = -kLead - 2; t < -1; ++t) copies();
-    // K of stages 0 and 1 landed, issued first in the first two of those iterations
-    pf::wait_vm<kCopies + 2 * kCopies * (kLead - 1)>();
+    // K of stages 0 and 1 landed: those of K stages 2 .. kLead and of V stages 0 .. kLead - 3 were issued after
+    pf::wait_vm<kCopies * (kLead - 1 + kLead - 2)>();
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the zeroed slot
     raw_barrier();
     // The scores and probabilities alternate between two register sets, so the iterations go in pairs;
@@ -601,7 +603,12 @@ __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParam
     next_k();
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     raw_barrier();                       // K stage 0 is read: its slot takes iteration -1's copies
-    copies();
+    off_v = off1;
+    next_stage();
+#pragma unroll
+    for (int k = 0; k < kCopies; ++k) copy_k(k);
+#pragma unroll
+    for (int k = 0; k < kCopies; ++k) copy_v(k, off_v);
     int t = 0;
     if (n & 1) {
 #pragma unroll
