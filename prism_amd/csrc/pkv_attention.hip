@@ -3065,19 +3065,29 @@ static size_t ws_bytes_prefill(int batch, int64_t R, int n_kv, int head_dim, int
 // Speculative verify on prefill_tile_kernel's two-wave form.  decode_lean_kernel's verify rows are one
 // serial chain per wave at one wave per SIMD, with a 1.8-2.4 us segment start per sequence and a
 // 7-8 us merge launch; this form runs six waves per CU and starts a range in about 2.5 us.  Per call,
-// five query rows, lean / tiles: 7B B = 8 25.3 / 20.1 us, B = 32 36.8 / 33.0, B = 64 72.9 / 69.7, B = 64
-// over a shared 2048-token prefix 55.8 / 50.0, 14B B = 16 36.7 / 36.6, B = 32 61.7 / 59.2.  Past one
-// (sequence, KV head) per CU the ranges no longer fit one round: 7B B = 128 124.6 / 133.2, shared 95.2 /
-// 96.2, so the rule ends there.
+// four query rows, lean / tiles: 7B, 8 sequences of 2000 keys 21.8 / 17.8 us, 32 of U{1..1000} 22.4 /
+// 18.2, 64 of 2000 65.6 / 60.4, 32 over a shared 8000-token prefix 86.6 / 57.5; 14B, 16 of 500 17.8 /
+// 17.1, 32 of U{1..1000} 28.0 / 23.1.
 // Its ranges are longer than decode_lean_kernel's shares, so fewer keys meet a running maximum of their
 // own, where P is exactly 1: rounded to bf16 once, P would be further off (7B, 2 to 12 short contexts:
 // 2.04e-3 from 64 bits on decode_lean_kernel, 2.24e-3 here).  It is a bf16 hi + lo pair instead, 1.66e-3
-// on every call, which is the output's own rounding; the second product of a stage costs 0 to 2%.
+// on every call, which is the output's own rounding; the second product costs a call 2 to 5%, and 10 to
+// 18% over a long shared prefix, whose keys come from the L2s.
 // It takes the calls of decode_lean_kernel's geometry of four KV heads at head_dim 128 with more than 16
-// query rows per KV head, unless a flag asks for a merge or a grid.  head_dim 64 and one or two KV heads
-// stay on decode_lean_kernel: there this form has been timed with P rounded once only (0.5B B = 64 40.0 /
-// 27.1 us, a TP-4 shard at B = 16 32.2 / 19.7), which is less exact than what they have.  Key ranges per
-// KV head: about one round of kVerifyPerCu workgroups per CU over all heads.
+// query rows per KV head, unless a flag asks for a merge or a grid, between three lines:
+//   one (sequence, KV head) per CU, past which the ranges no longer fit one round (7B, 128 sequences
+//     124.6 / 133.2);
+//   block tables of kVerifyKeys keys: a longer sequence has so many ranges that their merge is a chain of
+//     its own, and private keys come from memory, which decode_lean_kernel reads faster (7B, 8 lognormal
+//     contexts of up to 32000 39.2 / 43.6, 14B, 32 168 / 186).  Below the line the worst measured is a
+//     batch of equal lengths whose ranges leave a sixth of the round empty (40 of 6000 101 / 109);
+//   more than kVerifyFew keys in all where tables are of kVerifyShort: a few sequences of one or two
+//     hundred keys are one range each (7B, 8 of U{1..200} 11.8 / 12.7; 24 13.7 / 13.3).
+// head_dim 64 and one or two KV heads stay on decode_lean_kernel: there this form has been timed with P
+// rounded once only (0.5B B = 64 40.0 / 27.1 us, a TP-4 shard at B = 16 32.2 / 19.7), which is less exact
+// than what they have.  Key ranges per KV head: about one round of kVerifyPerCu workgroups per CU over
+// all heads.
+constexpr int64_t kVerifyKeys = 8192, kVerifyShort = 256, kVerifyFew = 4096;
 constexpr size_t kScratchBytes = size_t(48) << 20;  // pkv_decode_attn_noalloc's static scratch
 static int verify_target(int n_kv) {
   const int t = pf::kVerifyPerCu * device_cu_count() / n_kv;
@@ -3091,8 +3101,10 @@ static size_t ws_bytes_verify(int batch, int n_kv, int head_dim) {
 }
 // Only where the ranges fit the static scratch, so that a call takes the same kernel with and without
 // a workspace of its own.
-static bool use_verify_tiles(int batch, int n_kv, int head_dim, int R, int page_size, bool lean, int32_t flags) {
-  return lean && lean_geom(head_dim, n_kv) == kGeom128x4 && R > 16 && page_size >= pf::Geo<128>::TOK &&
+static bool use_verify_tiles(int batch, int n_kv, int head_dim, int R, int page_size, int max_blocks, bool lean,
+                             int32_t flags) {
+  const int64_t keys = int64_t(max_blocks) * page_size;  // a sequence's, by the table
+  return lean && keys <= kVerifyKeys && (keys > kVerifyShort || keys * batch > kVerifyFew) && lean_geom(head_dim, n_kv) == kGeom128x4 && R > 16 && page_size >= pf::Geo<128>::TOK &&
          (flags & ~PKV_DECODE_RESET_COUNTERS) == 0 && int64_t(batch) * n_kv <= device_cu_count() &&
          batch <= pf::kVerifyBatch &&
          ws_bytes_verify(batch, n_kv, head_dim) <= kScratchBytes;
@@ -3140,7 +3152,7 @@ extern "C" size_t pkv_decode_workspace_bytes(int32_t batch, int32_t s_q, int32_t
   if (use_lean_kernel(batch, head_dim, n_kv, R, page_size, split_tokens, 0)) {
     const size_t lean = ws_bytes_lean(lean_grid(0), R);
     need = lean > need ? lean : need;
-    if (use_verify_tiles(batch, n_kv, head_dim, R, page_size, true, 0)) {
+    if (use_verify_tiles(batch, n_kv, head_dim, R, page_size, max_blocks, true, 0)) {
       const size_t v = ws_bytes_verify(batch, n_kv, head_dim);
       need = v > need ? v : need;
     }
@@ -3249,7 +3261,7 @@ static int decode_attn(const char* fn, bool use_scratch, const void* q, int64_t 
   // may have read before the store.
   const bool lines = ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) |
                        uintptr_t(cache_page_stride) * 2) & 127) == 0;
-  const bool verify = (lines || !k_new) && use_verify_tiles(batch, n_kv, head_dim, R, page_size, lean, flags);
+  const bool verify = (lines || !k_new) && use_verify_tiles(batch, n_kv, head_dim, R, page_size, max_blocks, lean, flags);
   const size_t need = verify ? ws_bytes_verify(batch, n_kv, head_dim)
                       : lean ? ws_bytes_lean(grid, R)
                              : (ms > 1 ? ws_bytes(batch, R, n_kv, head_dim, ms) : 0);

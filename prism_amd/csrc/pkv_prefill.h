@@ -186,8 +186,7 @@ __device__ __forceinline__ VerifyPlan verify_plan(const AttnParams& p) {
 //
 // W waves own 32 W rows.  W = 2 (kSplit only) is speculative verify: one row block per (sequence, KV
 // head); each range appends the new rows it covers itself, before it copies them; P is a bf16 pair (two
-// PV products: the launch is bound by range starts and copies, 64 branches of one 2048-token prompt 49
-// -> 50 us a call).
+// PV products).
 template <int HD, int DEST, int W = pf::kWaves>
 __global__ __launch_bounds__(64 * W, 2) void prefill_tile_kernel(const AttnParams p) {
   using G = pf::Geo<HD>;

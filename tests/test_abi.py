@@ -141,6 +141,26 @@ def test_prefill_splits_where_ranges_pay(lib, sizes, splits):
     assert lib.pkv_prefill_workspace_bytes(*sizes) == want
 
 
+@pytest.mark.parametrize("batch,s_q,nh,nkv,hd,page,mb,tiles", [
+    (8, 5, 28, 4, 128, 256, 32, True), (8, 5, 28, 4, 128, 256, 33, False),    # 8192 keys
+    (16, 5, 28, 4, 128, 256, 1, False), (17, 5, 28, 4, 128, 256, 1, True),    # one page: 4096 keys in all
+    (2, 5, 28, 4, 128, 256, 2, True), (2, 2, 28, 4, 128, 256, 2, False),      # 14 query rows per KV head
+    (64, 5, 28, 4, 128, 256, 8, True), (65, 5, 28, 4, 128, 256, 8, False),    # one (sequence, KV head) per CU
+    (32, 5, 40, 8, 128, 256, 8, True), (33, 5, 40, 8, 128, 256, 8, False),
+    (4, 5, 14, 2, 128, 256, 8, False), (4, 5, 16, 4, 64, 256, 8, False), (4, 5, 28, 4, 128, 16, 100, False),
+])
+def test_verify_workspace_follows_the_rule(lib, batch, s_q, nh, nkv, hd, page, mb, tiles):
+    # 192 // (n_kv / 4) + batch key ranges per KV head of 64 rows x (128 + 2) floats, and two words per sequence
+    R = s_q * nh // nkv
+    need = 65536 + (768 // nkv + batch) * nkv * 64 * 130 * 4 + batch * 8
+    got = lib.pkv_decode_workspace_bytes(batch, s_q, nh, nkv, hd, page, mb, 0)
+    heads = 65536 + batch * nkv * -(-mb * page // 512) * R * (hd + 2) * 4   # the per-head kernel's, if it splits
+    others = max(65536 + 2 * 256 * 4 * R * 260, heads if mb * page > 512 else 0)
+    if page < 32:
+        others = heads
+    assert got == (max(need, others) if tiles else others)
+
+
 def test_copy_and_gather_argument_errors(lib):
     rc = lib.pkv_copy_pages(A16, A16, 2, A16, A16, None, 3, 1000, 1 << 18, 1024, 256, 10, 10, None, None)
     assert rc == _lib.PKV_EINVAL and "pkv_copy_pages" in lib.pkv_last_error().decode()

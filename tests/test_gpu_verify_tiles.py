@@ -145,3 +145,21 @@ def test_verify_appends_off_a_cache_line_keep_the_balanced_kernel(gpu, base, str
     again = prism_amd.flash_attn_with_kvcache(d["q"], kc, vc, **kw)
     assert_attn_close(again, ref, "off a cache line, no append")
     assert prism_amd.read_status(gpu) == 0
+
+
+@pytest.mark.parametrize("nh,ctx,tiles", [(28, [8100, 5], True), (28, [8300, 5], False), (28, [100] * 16, False),
+                                          (28, [100] * 17, True)])
+def test_verify_rule_by_table_width(gpu, nh, ctx, tiles):
+    """Both sides of the rule's lines: on the tile kernel the P of a call is a pair, on the balanced kernel
+    the call is bit-identical to the one a merge flag selects.  Either is within the tolerance."""
+    cpu, d = make_paged_case(gpu, batch=len(ctx), ctx=ctx, page_size=256, n_kv=4, n_heads=nh, head_dim=128, s_q=5,
+                             seed=len(ctx))
+    kw = dict(cache_seqlens=d["cache_seqlens"], block_table=d["block_table"], causal=True, shared_prefix_tokens=0)
+    a = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], **kw)
+    b = prism_amd.flash_attn_with_kvcache(d["q"], d["k_cache"], d["v_cache"], d["k"], d["v"], two_pass=True, **kw)
+    ref, _, _ = pa.flash_attn_with_kvcache_ref(cpu["q"], cpu["k_cache"], cpu["v_cache"], cpu["k"], cpu["v"],
+                                               cache_seqlens=cpu["cache_seqlens"], block_table=cpu["block_table"],
+                                               causal=True)
+    assert_attn_close(b, ref, "balanced")
+    assert_attn_close(a, ref, "the rule's choice")
+    assert torch.equal(a, b) is not tiles
