@@ -136,7 +136,7 @@ size_t pkv_decode_workspace_bytes(int32_t batch, int32_t s_q, int32_t n_heads, i
  * Without a merge flag or PKV_DECODE_GRID, the balanced kernel's head_dim 128 calls with n_kv a
  * multiple of 4, more than 16 rows per KV head and at most one (sequence, KV head) per CU run the
  * prefill tile kernel over ranges of keys instead, with fp32 partials and a second launch that merges
- * them, where max_blocks * page_size is at most 8192 keys, and above 256 or, times the batch, above
+ * them, where max_blocks * page_size is at most 10240 keys, and above 256 or, times the batch, above
  * 4096.  If the call appends, k_cache, v_cache and the page stride in bytes must also be multiples of
  * 128.  Calls that miss any of this keep the balanced kernel and its fp16 partials (below).
  * Otherwise a per-(sequence, KV head, split) kernel reduces split_tokens keys (a multiple of 32;

@@ -3079,15 +3079,16 @@ static size_t ws_bytes_prefill(int batch, int64_t R, int n_kv, int head_dim, int
 //     124.6 / 133.2);
 //   block tables of kVerifyKeys keys: a longer sequence has so many ranges that their merge is a chain of
 //     its own, and private keys come from memory, which decode_lean_kernel reads faster (7B, 8 lognormal
-//     contexts of up to 32000 39.2 / 43.6, 14B, 32 168 / 186).  Below the line the worst measured is a
-//     batch of equal lengths whose ranges leave a sixth of the round empty (40 of 6000 101 / 109);
+//     contexts of up to 32000 39.2 / 43.6, 14B, 32 168 / 186; 24 of up to 9200 52.7 / 53.8).  But 64
+//     sequences over a shared 8192-token prefix are worth it (149 / 97).  Below the line the worst measured
+//     is a batch of equal lengths whose ranges leave a sixth of the round empty (40 of 6000 101 / 109);
 //   more than kVerifyFew keys in all where tables are of kVerifyShort: a few sequences of one or two
 //     hundred keys are one range each (7B, 8 of U{1..200} 11.8 / 12.7; 24 13.7 / 13.3).
 // head_dim 64 and one or two KV heads stay on decode_lean_kernel: there this form has been timed with P
 // rounded once only (0.5B B = 64 40.0 / 27.1 us, a TP-4 shard at B = 16 32.2 / 19.7), which is less exact
 // than what they have.  Key ranges per KV head: about one round of kVerifyPerCu workgroups per CU over
 // all heads.
-constexpr int64_t kVerifyKeys = 8192, kVerifyShort = 256, kVerifyFew = 4096;
+constexpr int64_t kVerifyKeys = 10240, kVerifyShort = 256, kVerifyFew = 4096;
 constexpr size_t kScratchBytes = size_t(48) << 20;  // pkv_decode_attn_noalloc's static scratch
 static int verify_target(int n_kv) {
   const int t = pf::kVerifyPerCu * device_cu_count() / n_kv;

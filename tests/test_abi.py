@@ -142,7 +142,7 @@ def test_prefill_splits_where_ranges_pay(lib, sizes, splits):
 
 
 @pytest.mark.parametrize("batch,s_q,nh,nkv,hd,page,mb,tiles", [
-    (8, 5, 28, 4, 128, 256, 32, True), (8, 5, 28, 4, 128, 256, 33, False),    # 8192 keys
+    (8, 5, 28, 4, 128, 256, 40, True), (8, 5, 28, 4, 128, 256, 41, False),    # 10240 keys
     (16, 5, 28, 4, 128, 256, 1, False), (17, 5, 28, 4, 128, 256, 1, True),    # one page: 4096 keys in all
     (2, 5, 28, 4, 128, 256, 2, True), (2, 2, 28, 4, 128, 256, 2, False),      # 14 query rows per KV head
     (64, 5, 28, 4, 128, 256, 8, True), (65, 5, 28, 4, 128, 256, 8, False),    # one (sequence, KV head) per CU

@@ -147,7 +147,7 @@ def test_verify_appends_off_a_cache_line_keep_the_balanced_kernel(gpu, base, str
     assert prism_amd.read_status(gpu) == 0
 
 
-@pytest.mark.parametrize("nh,ctx,tiles", [(28, [8100, 5], True), (28, [8300, 5], False), (28, [100] * 16, False),
+@pytest.mark.parametrize("nh,ctx,tiles", [(28, [10200, 5], True), (28, [10300, 5], False), (28, [100] * 16, False),
                                           (28, [100] * 17, True)])
 def test_verify_rule_by_table_width(gpu, nh, ctx, tiles):
     """Both sides of the rule's lines: on the tile kernel the P of a call is a pair, on the balanced kernel
