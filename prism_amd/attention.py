@@ -341,9 +341,11 @@ def append_kv(k_cache, v_cache, k, v, cache_seqlens, block_table, *, status=None
 
 
 # Cascade attention is taken by itself (shared_prefix_tokens=None) from this many shared keys and
-# sequences on: at the Qwen2.5-7B verify shape (64 sequences, 5 query rows) the ordinary call is
-# faster at a 1792-key shared prefix (58.1-58.2 vs 59.8-60.7 us per layer) and the cascade 1.9x
-# faster at 7936; interpolated, the two cross near 2.2k shared keys.
+# sequences on.  The line dates from a slower ordinary call and is early for up to 64 sequences: us a
+# call at the Qwen2.5-7B verify shape (5 query rows, suffixes U{0..1000}), ordinary / cascade, at 2048,
+# 4096 and 8192 shared keys: 16 sequences 24.6 / 40.0, 29.7 / 41.9, 40.3 / 46.6; 32 30.7 / 46.7, 42.7 /
+# 51.9, 64.1 / 57.8; 64 47.9 / 57.5, 69.6 / 65.8, 115 / 84.8; 96 (the balanced kernel) 77.3 / 70.7, 115 /
+# 83.0, 194 / 109.
 AUTO_CASCADE_MIN_TOKENS = 2048
 AUTO_CASCADE_MIN_BATCH = 4
 

@@ -16,10 +16,11 @@
 // two of K and two of V per wave), through a ring of 4 slots of K and one of 4 of V (3 each in the
 // two-wave form), with counted vmcnt waits and one raw barrier per stage.
 //
-// What bounds it: the matrix pipe at 33 cycles per 32x32x16 product (16 products per tile and wave)
-// beside some 60 vector instructions of softmax and 24 LDS reads, and above that the card's power: a
-// register-only loop of these products on random data holds 1.53 GHz on 256 CUs (2.1 on constants).
-// A wave issues in order, about one instruction per 4.4 cycles, so its iteration over stage t mixes
+// What bounds it: the matrix pipe at 33 cycles per 32x32x16 product (16 products per stage and wave)
+// beside 79 other vector instructions and 24 LDS reads.  The pipe is busy 46% of a launch of 1280
+// workgroups; a wave issues 47% of its time, waits for a pipe 34% (the other wave of its SIMD has it)
+// and at the barrier and copies 19%.  Power is not the limit yet: a register-only loop of these products
+// on random data holds 1.53 GHz on 256 CUs, the launch runs at about 1.95.  A wave issues in order, about one instruction per 4.4 cycles, so its iteration over stage t mixes
 // three stages to keep both pipes fed, in straight-line code (a taken branch costs 50-100 cycles of
 // instruction fetch; rare work sits out of line):
 //   phase A: S^T products of stage t + 1, with the first half of stage t's exponentials between them,
@@ -29,8 +30,9 @@
 //            drifts the two waves of a SIMD into opposite phases (4096-token 7B prompt 154 -> 148 us).
 // The copies of a stage go out one at a time through both phases (all in phase A: 146 -> 139 us).
 // Per call: head_dim 64, 4 prompts of 1000 tokens, 93 -> 35 us (it replaces per-wave tiles held in
-// registers); head_dim 128, one 4096-token 7B prompt 136 -> 133 us, 8 x 512 14B chunks onto
-// prefixes U{0..4096} 169 -> 162 us, 150 tokens onto 3500 (36 workgroups) 104 -> 70 us.
+// registers); head_dim 128, one 4096-token 7B prompt 136 -> 131 us, 8 x 512 14B chunks onto
+// prefixes U{0..4096} 169 -> 160 us, 150 tokens onto 3500 (36 workgroups) 104 -> 70 us.  Captured prompts
+// of one to three stages take 0.1 to 0.6 us more than with 16x16x32 products.
 namespace pf {
 
 template <int HD_>
