@@ -20,9 +20,10 @@
 // beside 79 other vector instructions and 24 LDS reads.  The pipe is busy 46% of a launch of 1280
 // workgroups; a wave issues 47% of its time, waits for a pipe 34% (the other wave of its SIMD has it)
 // and at the barrier and copies 19%.  Power is not the limit yet: a register-only loop of these products
-// on random data holds 1.53 GHz on 256 CUs, the launch runs at about 1.95.  A wave issues in order, about one instruction per 4.4 cycles, so its iteration over stage t mixes
-// three stages to keep both pipes fed, in straight-line code (a taken branch costs 50-100 cycles of
-// instruction fetch; rare work sits out of line):
+// on random data holds 1.53 GHz on 256 CUs, the launch runs at about 1.95.  A wave issues in order, about
+// one instruction per 4.4 cycles, so its iteration over stage t mixes three stages to keep both pipes
+// fed, in straight-line code (a taken branch costs 50-100 cycles of instruction fetch; rare work sits out
+// of line):
 //   phase A: S^T products of stage t + 1, with the first half of stage t's exponentials between them,
 //            while stage t - 1's V operands arrive from LDS;
 //   phase B: PV products of stage t - 1, with the second half and the next stage's score maxima between
